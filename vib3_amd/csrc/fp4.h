@@ -55,6 +55,25 @@ __device__ __forceinline__ float e8m0_inv(uint32_t e) {
   return e == 0 ? __builtin_huge_valf() : __uint_as_float((254u - e) << 23);
 }
 
+// Eight f32 values as E2M1 codes of the scale 2^(e - 127), value j in nibble j. The conversion
+// instruction gives e2m1_rne(v * e8m0_inv(e)) for every f32 bit pattern, NaN and infinities
+// included (compared exhaustively, for e from 1 to 253); e = 0 stands for a group whose values are
+// zeros or NaNs, whose codes do not depend on a scale (f32 input whose maximum is positive and still
+// below the E8M0 range is the caller's to handle: there every code is 7 by v * inf).
+__device__ __forceinline__ uint32_t quantize8(const float (&v)[8], uint32_t e) {
+  const float scale = e == 0 ? 1.0f : __uint_as_float(e << 23);
+  uint32_t c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, v[0], v[1], scale, 0);
+  c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v[2], v[3], scale, 1);
+  c = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v[4], v[5], scale, 2);
+  return __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(c, v[6], v[7], scale, 3);
+}
+
+// The low four nibbles of x, one per byte.
+__device__ __forceinline__ uint32_t spread_nibbles(uint32_t x) {
+  x = (x | (x << 8)) & 0x00ff00ffu;
+  return (x | (x << 4)) & 0x0f0f0f0fu;
+}
+
 // e^x by Cody-Waite reduction x = n ln2 + r (ln2 split in a 15-bit head and a tail, so n * head
 // is exact) and the degree-7 Taylor polynomial of e^r on |r| <= ln2 / 2 in Horner form, then
 // ldexp. Every operation is a single IEEE rounding (no contraction), so the oracle's C version
