@@ -441,8 +441,9 @@ int vib3_launch_fused_swiglu_nvfp4_f32out(const void *input, const void *up_weig
 int vib3_launch_repack_weights_inplace(void *weight_data_ptr, long long weight_data_bytes,
                                        void *stream);
 
-/* cuda_ffi.rs:718 (kernels.cu:4227-4262): row-major split-half [M][K/2] -> tiled, through
- * temp_buf (M*K/2 bytes), then copied back. M % 16 == 0, K % 64 == 0. */
+/* cuda_ffi.rs:718 (kernels.cu:4227-4262): row-major split-half [M][K/2] -> tiled, in place;
+ * above K = 16384 through temp_buf (M*K/2 bytes, whose contents are not defined afterwards) and
+ * copied back. M % 16 == 0, K % 64 == 0. */
 int vib3_launch_repack_row_to_tiled(void *weight_data_ptr, void *temp_buf, int M, int K,
                                     void *stream);
 
