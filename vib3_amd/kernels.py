@@ -66,7 +66,7 @@ def _act_dt(t: torch.Tensor, name: str) -> int:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.current_stream(t.get_device())
 
 
 def _need_int4(weight_dtype: int) -> None:

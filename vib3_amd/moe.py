@@ -231,7 +231,7 @@ class MoeInt4Layer:
             if residual.dtype != torch.float32 or residual.numel() != self.bank.shape.hidden:
                 raise TypeError("residual must be f32 [hidden]")
             desc.residual = residual.data_ptr()
-        st = (stream or torch.cuda.current_stream(x.device)).cuda_stream
+        st = stream.cuda_stream if stream else _lib.current_stream(x.get_device())
         rc = _lib.load().vib3_launch_moe_int4_layer(desc, st)
         if rc != 0:
             raise _lib.Vib3Error("vib3_launch_moe_int4_layer", rc)

@@ -115,7 +115,7 @@ class MoeMxfp4Batch:
 
     def launch(self, x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor) -> torch.Tensor:
         d = self.desc(x, ids, weights)
-        st = torch.cuda.current_stream(self.bank.device).cuda_stream
+        st = _lib.current_stream(self.bank.buf.get_device())
         rc = _lib.load().vib3_launch_moe_mxfp4_batched(d, st)
         if rc:
             raise _lib.Vib3Error("vib3_launch_moe_mxfp4_batched", rc)
