@@ -33,6 +33,8 @@ namespace {
 
 enum { kLayRowSplit = 0, kLayTiled = 1, kLaySeq = 2 };
 
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+
 struct PageGemvArgs {
   const uint8_t* act;     // split-half activation codes [K/32][16], or null: quantize x
   const uint8_t* act_sc;  // [K/32] E8M0
@@ -43,31 +45,22 @@ struct PageGemvArgs {
   int K, M;
 };
 
-// Sequential 16 bytes (value 2j low, 2j + 1 high) as split-half (byte j: value j | value j + 16).
-__device__ __forceinline__ uint4 seq_to_split(uint4 v) {
-  const uint32_t in[4] = {v.x, v.y, v.z, v.w};
-  uint32_t o[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int j = 0; j < 8; j++) {
-    const uint32_t s0 = (in[j >> 2] >> (8 * (j & 3))) & 0xff;
-    const uint32_t s1 = (in[(j + 8) >> 2] >> (8 * ((j + 8) & 3))) & 0xff;
-    o[(2 * j) >> 2] |= ((s0 & 0x0f) | ((s1 & 0x0f) << 4)) << (8 * ((2 * j) & 3));
-    o[(2 * j + 1) >> 2] |= ((s0 >> 4) | (s1 & 0xf0)) << (8 * ((2 * j + 1) & 3));
-  }
-  return make_uint4(o[0], o[1], o[2], o[3]);
-}
-
-// One group's 16 split-half bytes as the LDS pair layout group_dot reads.
-__device__ __forceinline__ void put_group(uint4* pairs, int* ex, int g, uint4 w, int e) {
-  f16x2 p[16];
-  decode_group(w, p);
-#pragma unroll
-  for (int q = 0; q < 4; q++)
-    pairs[(size_t)g * 4 + q] =
-        make_uint4(__builtin_bit_cast(uint32_t, p[4 * q]), __builtin_bit_cast(uint32_t, p[4 * q + 1]),
-                   __builtin_bit_cast(uint32_t, p[4 * q + 2]), __builtin_bit_cast(uint32_t, p[4 * q + 3]));
-  ex[g] = e;
-}
+// How both kernels split a page (one launch reads at most a few megabytes, so they are bound by
+// the round trips of a launch, not by bandwidth: every load a wave needs goes out at once, and the
+// page is spread over as many waves as it has row groups).
+//   * A row is read by L lanes, R = 64 / L rows by a wave; lane `sub` of a row takes the 32-value
+//     groups sub, sub + L, ... (16 bytes each, so a load instruction reads 16 L contiguous bytes of
+//     each row). L is the smallest of 16, 32 and 64 for which a row takes one pass of kJ groups per
+//     lane (K <= 2048, 4096, 8192); above that L = 64 and the row takes several passes.
+//   * The activation groups a lane multiplies are the same for every row, so they are decoded into
+//     registers straight from memory: no staging, no barrier. (Decoding the whole activation into
+//     LDS in 16-row workgroups used 33 of the 256 CUs for a 520-row page and waited for two barriers
+//     and 56 dependent steps per lane.)
+//   * Waves stride over the row groups, the next group's weights loading while one is reduced.
+// Traced: 520-row gate/up page pair at K = 7168 (4.2 MB) 12.2 -> 5.1 us (f32 input quantized in the
+// kernel: 36.7 -> 6.8), 1820-row down page at K = 2048 (2.1 MB) 4.9 -> 4.2 us, a pair of 14336 rows
+// at K = 4096 (66 MB) 19.6 -> 14.1 us.
+constexpr int kJ = 4;
 
 // Bytes of group g of row r in layout LAY.
 template <int LAY>
@@ -77,62 +70,201 @@ __device__ __forceinline__ const uint8_t* group_ptr(const uint8_t* w, int r, int
   return w + (size_t)r * (K / 2) + (size_t)g * 16;
 }
 
-// Workgroup = 16 rows, 16 lanes per row (a lane takes groups l, l + 16, ...), the activation
-// staged once per workgroup in LDS as decoded pairs and exponents.
-template <int LAY, bool FULL, int NS>
-__global__ __launch_bounds__(256) void k_fp4_page_gemv(PageGemvArgs a) {
-  extern __shared__ uint4 lds[];
-  const int G = a.K / 32, tid = (int)threadIdx.x, lane = lane_id();
-  uint4* pairs = lds;                      // [G][4]
-  int* ex = (int*)(lds + (size_t)G * 4);   // [G]
-  if (a.act) {
-    for (int g = tid; g < G; g += 256) put_group(pairs, ex, g, *(const uint4*)(a.act + (size_t)g * 16), a.act_sc[g]);
-  } else {
-    // the activation quantizer's rule (kernels.cu:3193-3240, inline at :3418-3470): a 32-lane
-    // half-wave per group, E8M0 of its absolute maximum, codes rounded to nearest even
-    uint8_t* codes = (uint8_t*)(ex + G);  // [G][16]
-    int* es = (int*)(codes + (size_t)G * 16 + 16);
-    es = (int*)(((uintptr_t)es + 3) & ~(uintptr_t)3);
-    for (int base = 0; base < G * 32; base += 256) {
-      const int i = base + tid;
-      const float v = i < a.K ? a.x[i] : 0.0f;
-      float amax = fabsf(v);
+// One pass's weights of a row group: code words and scales of NS matrices.
+template <int NS>
+struct PageStep {
+  uint4 w[NS][kJ];
+  uint16_t q[NS][kJ];
+};
+
+// Groups past the row end re-read its last group (no branch around the loads).
+template <int LAY, int NS, int L>
+__device__ __forceinline__ void page_issue(PageStep<NS>& b, const uint8_t* const (&w)[2],
+                                           const uint16_t* const (&s)[2], int row, int pass, int K,
+                                           int G, int sc_shift) {
+  const int sub = lane_id() % L;
 #pragma unroll
-      for (int m = 1; m < 32; m <<= 1) amax = fmaxf(amax, __shfl_xor(amax, m));
-      const uint32_t e = e8m0_of_amax(amax);
-      const float inv = amax == 0.0f ? 0.0f : e8m0_inv(e);
-      const uint32_t code = e2m1_rne(v * inv);
-      const uint32_t hi = (uint32_t)__shfl(code, (lane & ~31) + (lane & 15) + 16);
-      const int g = i >> 5, j = i & 31;
-      if (j < 16 && g < G) codes[(size_t)g * 16 + j] = (uint8_t)(code | (hi << 4));
-      if (j == 0 && g < G) es[g] = (int)e;
-    }
-    __syncthreads();
-    for (int g = tid; g < G; g += 256) put_group(pairs, ex, g, *(const uint4*)(codes + (size_t)g * 16), es[g]);
-  }
-  __syncthreads();
-  const int gl = tid & 15, row = (int)blockIdx.x * 16 + (tid >> 4);
-  const int rc = row < a.M ? row : a.M - 1;
-  double acc[NS];
-#pragma unroll
-  for (int m = 0; m < NS; m++) acc[m] = 0.0;
-  for (int g = gl; g < G; g += 16) {
-    const double ea = pow2d(ex[g] - 127);
+  for (int j = 0; j < kJ; j++) {
+    if (pass * L * kJ + L * j >= G) break;  // (wave-uniform)
+    const int g = min((pass * kJ + j) * L + sub, G - 1);
 #pragma unroll
     for (int m = 0; m < NS; m++) {
-      uint4 w = *(const uint4*)group_ptr<LAY>(a.w[m], rc, g, a.K);
-      if (LAY == kLaySeq) w = seq_to_split(w);
-      const uint16_t sw = a.s[m][(size_t)rc * G + g];
-      const double ws = FULL ? (double)bf16_to_f32(sw) : pow2d((int)((sw >> 7) & 0xff) - 127);
-      acc[m] = fma((double)group_dot(w, pairs + (size_t)g * 4), ws * ea, acc[m]);
+      b.w[m][j] = ld_stream(group_ptr<LAY>(w[m], row, g, K));
+      b.q[m][j] = ld_u16(s[m] + (size_t)row * (G >> sc_shift) + (g >> sc_shift));
     }
   }
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, 0xf, 0xf, true);
+  return __longlong_as_double(((long long)hi << 32) | (uint32_t)lo);
+}
+
+// Sum over a row's L lanes (every lane gets it).
+template <int L>
+__device__ __forceinline__ double row_sum(double v) {
+  v += dpp_d<0xB1>(v);
+  v += dpp_d<0x4E>(v);
+  v += dpp_d<0x141>(v);
+  v += dpp_d<0x140>(v);
+  if (L >= 32) v += shfl_xor_d(v, 16);
+  if (L >= 64) v += shfl_xor_d(v, 32);
+  return v;
+}
+template <int L>
+__device__ __forceinline__ float row_sum(float v) {
+  v += dpp<0xB1>(v);
+  v += dpp<0x4E>(v);
+  v += dpp<0x141>(v);
+  v += dpp<0x140>(v);
+  if (L >= 32) v += __shfl_xor(v, 16);
+  if (L >= 64) v += __shfl_xor(v, 32);
+  return v;
+}
+
+// 32 consecutive f32 values (16-byte loads where `vec`).
+__device__ __forceinline__ void load32(const float* x, bool vec, float (&v)[32]) {
+  if (vec) {
 #pragma unroll
-  for (int m = 0; m < NS; m++)
+    for (int i = 0; i < 8; i++) {
+      const float4 t = ((const float4*)x)[i];
+      v[4 * i] = t.x; v[4 * i + 1] = t.y; v[4 * i + 2] = t.z; v[4 * i + 3] = t.w;
+    }
+  } else {
 #pragma unroll
-    for (int o = 1; o < 16; o <<= 1) acc[m] += shfl_xor_d(acc[m], o);
-  if (gl == 0 && row < a.M)
-    a.out[row] = NS == 1 ? (float)acc[0] : swiglu_fp4((float)acc[1], (float)acc[0]);
+    for (int i = 0; i < 32; i++) v[i] = x[i];
+  }
+}
+
+// The activation quantizer's rule (kernels.cu:3193-3240, inline at :3418-3470) for one group:
+// E8M0 of the absolute maximum, codes rounded to nearest even, in sequential order.
+__device__ __forceinline__ uint4 quantize_group_seq(const float (&v)[32], int& e_out) {
+  float amax = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 32; i++) amax = fmaxf(amax, fabsf(v[i]));
+  const uint32_t e = e8m0_of_amax(amax);
+  e_out = (int)e;
+  uint32_t o[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float t[8] = {v[8 * i], v[8 * i + 1], v[8 * i + 2], v[8 * i + 3],
+                        v[8 * i + 4], v[8 * i + 5], v[8 * i + 6], v[8 * i + 7]};
+    o[i] = quantize8(t, e);
+  }
+  if (e == 0 && amax > 0.0f) {  // below the E8M0 range: v * inf, as k_fp4_quant_act
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      o[i] = 0;
+#pragma unroll
+      for (int j = 0; j < 8; j++) o[i] |= e2m1_rne(v[8 * i + j] * e8m0_inv(0)) << (4 * j);
+    }
+  }
+  return make_uint4(o[0], o[1], o[2], o[3]);
+}
+
+// Block-scaled GEMV of NS matrices (NS = 2: up and gate, SwiGLU). ONE: a row is one pass.
+// Sequential weights meet a sequential activation: with f32 input the workgroup quantizes it into
+// LDS first (one group per thread), in the order the weights have.
+template <int LAY, bool FULL, int NS, int L, bool ONE>
+__global__ __launch_bounds__(256) void k_fp4_page_rows(PageGemvArgs a) {
+  extern __shared__ uint4 lds[];
+  constexpr int R = kWave / L;
+  const int G = a.K / 32, M = a.M, lane = lane_id(), sub = lane % L, rr = lane / L;
+  const int wpb = (int)(blockDim.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int groups = (M + R - 1) / R, stride = (int)gridDim.x * wpb;
+  int rg = (int)blockIdx.x * wpb + wave;
+  const uint8_t* const w[2] = {a.w[0], a.w[1]};
+  const uint16_t* const s[2] = {a.s[0], a.s[1]};
+  auto row_of = [&](int q) { return min(q * R + rr, M - 1); };
+  PageStep<NS> A, B;
+  const int passes = ONE ? 1 : (G + L * kJ - 1) / (L * kJ);
+  if (LAY != kLaySeq) page_issue<LAY, NS, L>(A, w, s, row_of(rg), 0, a.K, G, 0);
+  const uint8_t* codes = a.act;
+  int* es = nullptr;
+  if (LAY == kLaySeq) {
+    es = (int*)(lds + G);
+    const bool vec = ((uintptr_t)a.x & 15) == 0;
+    for (int g = (int)threadIdx.x; g < G; g += (int)blockDim.x) {
+      float v[32];
+      load32(a.x + (size_t)g * 32, vec, v);
+      int e;
+      lds[g] = quantize_group_seq(v, e);
+      es[g] = e;
+    }
+    __syncthreads();
+    page_issue<LAY, NS, L>(A, w, s, row_of(rg), 0, a.K, G, 0);
+  }
+  f16x2 xp[kJ][16];
+  int ex[kJ];
+  auto load_act = [&](int pass) {
+#pragma unroll
+    for (int j = 0; j < kJ; j++) {
+      if (pass * L * kJ + L * j >= G) break;
+      const int g0 = (pass * kJ + j) * L + sub, g = min(g0, G - 1);
+      const uint4 c = LAY == kLaySeq ? lds[g] : *(const uint4*)(codes + (size_t)g * 16);
+      ex[j] = LAY == kLaySeq ? es[g] : (int)a.act_sc[g];
+      // a group past the row end counts as zeros
+      decode_group(g0 < G ? c : make_uint4(0u, 0u, 0u, 0u), xp[j]);
+    }
+  };
+  double acc[NS];
+  auto reduce = [&](const PageStep<NS>& b, int pass) {
+#pragma unroll
+    for (int j = 0; j < kJ; j++) {
+      if (pass * L * kJ + L * j >= G) break;
+#pragma unroll
+      for (int m = 0; m < NS; m++) {
+        f16x2 wp[16];
+        decode_group(b.w[m][j], wp);
+        float d = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; i++) d = __builtin_amdgcn_fdot2(wp[i], xp[j][i], d, false);
+        const int ew = (b.q[m][j] >> 7) & 0xff;
+        const double sc = FULL ? (double)bf16_to_f32(b.q[m][j]) * pow2d(ex[j] - 127)
+                               : pow2d(ew + ex[j] - 254);
+        // a group past the row end: d = 0, and its scale may be anything
+        const double t = fma((double)d, sc, acc[m]);
+        acc[m] = (pass * kJ + j) * L + sub < G ? t : acc[m];
+      }
+    }
+  };
+  auto finish = [&](int q) {
+    double t[NS];
+#pragma unroll
+    for (int m = 0; m < NS; m++) t[m] = row_sum<L>(acc[m]);
+    const int row = q * R + rr;
+    if (sub == 0 && row < M)
+      a.out[row] = NS == 1 ? (float)t[0] : swiglu_fp4((float)t[NS - 1], (float)t[0]);
+  };
+  if (ONE) {
+    load_act(0);
+    for (;; ) {
+      // the next row group (past the end: the last row again, dropped)
+      page_issue<LAY, NS, L>(B, w, s, row_of(min(rg + stride, groups)), 0, a.K, G, 0);
+#pragma unroll
+      for (int m = 0; m < NS; m++) acc[m] = 0.0;
+      reduce(A, 0);
+      finish(rg);
+      rg += stride;
+      if (rg >= groups) break;
+      A = B;
+    }
+  } else {
+    for (; rg < groups; rg += stride) {
+#pragma unroll
+      for (int m = 0; m < NS; m++) acc[m] = 0.0;
+      for (int p = 0; p < passes; p++) {
+        if (p > 0 || rg >= stride) page_issue<LAY, NS, L>(A, w, s, row_of(rg), p, a.K, G, 0);
+        load_act(p);
+        reduce(A, p);
+      }
+      finish(rg);
+    }
+  }
 }
 
 struct ScalarArgs {
@@ -143,54 +275,106 @@ struct ScalarArgs {
   int K, M, bs_shift;     // block size 32 << bs_shift... as a shift of 32-value groups
 };
 
-__device__ __forceinline__ float e2m1_lut(uint32_t q) {
-  const float m[8] = {0.0f, 0.5f, 1.0f, 1.5f, 2.0f, 3.0f, 4.0f, 6.0f};
-  const float v = m[q & 7];
-  return (q & 8) ? -v : v;
-}
-
 // out[r] = sum_k x[k] * e2m1(W[r][k]) * bf16(s[r][k / bs]) in f32: per 32-value group the
 // products x * e2m1 summed with fused multiply-adds, then times the block scale into the row
 // sum; SwiGLU (NS = 2: up, gate) as the reference's epilogue silu(g) * u with
-// silu(g) = g / (1 + e^-g) (kernels.cu:580-582, :2027-2028). x staged in LDS as f32.
-template <bool IN16, bool OUT16, int NS>
-__global__ __launch_bounds__(256) void k_nvfp4_scalar(ScalarArgs a) {
-  extern __shared__ float xs[];
-  const int tid = (int)threadIdx.x, G = a.K / 32;
-  for (int i = tid; i < a.K; i += 256)
-    xs[i] = IN16 ? f16_to_f32(((const uint16_t*)a.x)[i]) : ((const float*)a.x)[i];
-  __syncthreads();
-  const int gl = tid & 15, row = (int)blockIdx.x * 16 + (tid >> 4);
-  const int rc = row < a.M ? row : a.M - 1;
-  const int nb = G >> a.bs_shift;
-  float acc[NS];
+// silu(g) = g / (1 + e^-g) (kernels.cu:580-582, :2027-2028). The lane's x groups stay in registers
+// as f32; split as above (a 520-row pair at K = 7168: 90 -> 8.0 us).
+template <bool IN16, bool OUT16, int NS, int L, bool ONE>
+__global__ __launch_bounds__(256) void k_nvfp4_scalar_rows(ScalarArgs a) {
+  constexpr int R = kWave / L;
+  const int G = a.K / 32, M = a.M, lane = lane_id(), sub = lane % L, rr = lane / L;
+  const int wpb = (int)(blockDim.x >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int groups = (M + R - 1) / R, stride = (int)gridDim.x * wpb;
+  const uint8_t* const w[2] = {a.w[0], a.w[1]};
+  const uint16_t* const s[2] = {a.s[0], a.s[1]};
+  const int passes = ONE ? 1 : (G + L * kJ - 1) / (L * kJ);
+  const bool vec = ((uintptr_t)a.x & 15) == 0;
+  PageStep<NS> A;
+  float xv[kJ][32];
+  auto load_x = [&](int pass) {
 #pragma unroll
-  for (int m = 0; m < NS; m++) acc[m] = 0.0f;
-  for (int g = gl; g < G; g += 16) {
+    for (int j = 0; j < kJ; j++) {
+      if (pass * L * kJ + L * j >= G) break;
+      const int g0 = (pass * kJ + j) * L + sub, g = min(g0, G - 1);
+      if (!IN16) {
+        load32((const float*)a.x + (size_t)g * 32, vec, xv[j]);
+      } else {
+        const uint16_t* p = (const uint16_t*)a.x + (size_t)g * 32;
 #pragma unroll
-    for (int m = 0; m < NS; m++) {
-      const uint4 w = *(const uint4*)(a.w[m] + (size_t)rc * (a.K / 2) + (size_t)g * 16);
-      const uint32_t wd[4] = {w.x, w.y, w.z, w.w};
-      float p = 0.0f;
+        for (int i = 0; i < 4; i++) {
+          uint4 t;
+          if (vec) t = ((const uint4*)p)[i];
+          else __builtin_memcpy(&t, p + 8 * i, 16);
+          const uint32_t tw[4] = {t.x, t.y, t.z, t.w};
 #pragma unroll
-      for (int i = 0; i < 16; i++) {
-        const uint32_t b = (wd[i >> 2] >> (8 * (i & 3))) & 0xff;
-        p = __builtin_fmaf(xs[g * 32 + 2 * i], e2m1_lut(b & 15), p);
-        p = __builtin_fmaf(xs[g * 32 + 2 * i + 1], e2m1_lut(b >> 4), p);
+          for (int k = 0; k < 8; k++) xv[j][8 * i + k] = f16_to_f32((uint16_t)(tw[k >> 1] >> (16 * (k & 1))));
+        }
       }
-      acc[m] = __builtin_fmaf(p, bf16_to_f32(a.s[m][(size_t)rc * nb + (g >> a.bs_shift)]), acc[m]);
+    }
+  };
+  float acc[NS];
+  auto reduce = [&](const PageStep<NS>& b, int pass) {
+#pragma unroll
+    for (int j = 0; j < kJ; j++) {
+      if (pass * L * kJ + L * j >= G) break;
+#pragma unroll
+      for (int m = 0; m < NS; m++) {
+        const uint32_t wd[4] = {b.w[m][j].x, b.w[m][j].y, b.w[m][j].z, b.w[m][j].w};
+        float p = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const f32x2 v0 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wd[i], 1.0f, 0);
+          const f32x2 v1 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wd[i], 1.0f, 1);
+          const f32x2 v2 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wd[i], 1.0f, 2);
+          const f32x2 v3 = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(wd[i], 1.0f, 3);
+          const float e[8] = {v0[0], v0[1], v1[0], v1[1], v2[0], v2[1], v3[0], v3[1]};
+#pragma unroll
+          for (int k = 0; k < 8; k++) p = __builtin_fmaf(xv[j][8 * i + k], e[k], p);
+        }
+        const float t = __builtin_fmaf(p, bf16_to_f32(b.q[m][j]), acc[m]);
+        acc[m] = (pass * kJ + j) * L + sub < G ? t : acc[m];
+      }
+    }
+  };
+  for (int rg = (int)blockIdx.x * wpb + wave, first = rg; rg < groups; rg += stride) {
+#pragma unroll
+    for (int m = 0; m < NS; m++) acc[m] = 0.0f;
+    for (int p = 0; p < passes; p++) {
+      page_issue<kLaySeq, NS, L>(A, w, s, min(rg * R + rr, M - 1), p, a.K, G, a.bs_shift);
+      if (!ONE || rg == first) load_x(p);
+      reduce(A, p);
+    }
+    float t[NS];
+#pragma unroll
+    for (int m = 0; m < NS; m++) t[m] = row_sum<L>(acc[m]);
+    const int row = rg * R + rr;
+    if (sub == 0 && row < M) {
+      const float v = NS == 1 ? t[0] : (t[NS - 1] / (1.0f + expf(-t[NS - 1]))) * t[0];
+      if (OUT16) ((uint16_t*)a.out)[row] = f32_to_f16_bits(v);
+      else ((float*)a.out)[row] = v;
     }
   }
-#pragma unroll
-  for (int m = 0; m < NS; m++)
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) acc[m] += __shfl_xor(acc[m], o);
-  if (gl == 0 && row < a.M) {
-    float v = acc[0];
-    if (NS == 2) v = (acc[1] / (1.0f + expf(-acc[1]))) * acc[0];
-    if (OUT16) ((uint16_t*)a.out)[row] = f32_to_f16_bits(v);
-    else ((float*)a.out)[row] = v;
-  }
+}
+
+// Launch shape for M rows of G groups: L lanes per row (see above), and one wave per row group up
+// to eight per CU, two to a workgroup while that spreads a page over more CUs.
+struct PageShape {
+  int L;
+  bool one;
+  unsigned grid, block;
+};
+PageShape page_shape(int M, int G) {
+  PageShape p{};
+  p.L = G <= 16 * kJ ? 16 : G <= 32 * kJ ? 32 : 64;
+  p.one = G <= p.L * kJ;
+  const int groups = (M + kWave / p.L - 1) / (kWave / p.L);
+  const int waves = groups < 8 * device_cus() ? groups : 8 * device_cus();
+  const int wpb = waves <= 4 * device_cus() ? 2 : 4;
+  p.block = 64u * wpb;
+  p.grid = (unsigned)((waves + wpb - 1) / wpb);
+  return p;
 }
 
 int page_gemv(int lay, bool full, int ns, const void* act, const void* act_sc, const float* x,
@@ -204,16 +388,25 @@ int page_gemv(int lay, bool full, int ns, const void* act, const void* act_sc, c
     return VIB3_ERR_BAD_POINTER;
   if (M == 0) return 0;
   const int G = K / 32;
-  const size_t lds = (size_t)G * 68 + (act ? 0 : (size_t)G * 20 + 32);
-  if (lds > 65536) return VIB3_ERR_UNSUPPORTED;
+  // K's limit (30816, or 23808 with f32 input): the whole decoded activation in 64 KB
+  if ((size_t)G * 68 + (act ? 0 : (size_t)G * 20 + 32) > 65536) return VIB3_ERR_UNSUPPORTED;
   PageGemvArgs a{};
   a.act = (const uint8_t*)act; a.act_sc = (const uint8_t*)act_sc; a.x = x;
   a.w[0] = (const uint8_t*)w0; a.s[0] = (const uint16_t*)s0;
   a.w[1] = (const uint8_t*)w1; a.s[1] = (const uint16_t*)s1;
   a.out = (float*)out; a.K = K; a.M = M;
-  const dim3 grid((unsigned)((M + 15) / 16)), block(256);
+  const PageShape p = page_shape(M, G);
+  const unsigned lds = act ? 0u : (unsigned)G * 20u;
   hipStream_t st = (hipStream_t)stream;
-#define VIB3_PAGE_GEMV(L, F, N) hipLaunchKernelGGL((k_fp4_page_gemv<L, F, N>), grid, block, (unsigned)lds, st, a)
+#define VIB3_PAGE_L(LY, F, N, LL, O) \
+  hipLaunchKernelGGL((k_fp4_page_rows<LY, F, N, LL, O>), dim3(p.grid), dim3(p.block), lds, st, a)
+#define VIB3_PAGE_GEMV(LY, F, N)                        \
+  do {                                                  \
+    if (p.L == 16) VIB3_PAGE_L(LY, F, N, 16, true);     \
+    else if (p.L == 32) VIB3_PAGE_L(LY, F, N, 32, true); \
+    else if (p.one) VIB3_PAGE_L(LY, F, N, 64, true);    \
+    else VIB3_PAGE_L(LY, F, N, 64, false);              \
+  } while (0)
   if (lay == kLayRowSplit && !full && ns == 1) VIB3_PAGE_GEMV(kLayRowSplit, false, 1);
   else if (lay == kLayRowSplit && !full && ns == 2) VIB3_PAGE_GEMV(kLayRowSplit, false, 2);
   else if (lay == kLayRowSplit && full && ns == 1) VIB3_PAGE_GEMV(kLayRowSplit, true, 1);
@@ -222,6 +415,7 @@ int page_gemv(int lay, bool full, int ns, const void* act, const void* act_sc, c
   else if (lay == kLaySeq && !full && ns == 2) VIB3_PAGE_GEMV(kLaySeq, false, 2);
   else return VIB3_ERR_UNSUPPORTED;
 #undef VIB3_PAGE_GEMV
+#undef VIB3_PAGE_L
   VIB3_RETURN_LAUNCH();
 }
 
@@ -237,15 +431,25 @@ int scalar_gemv(bool in16, bool out16, int ns, const void* x, const void* w0, co
   a.x = x; a.w[0] = (const uint8_t*)w0; a.s[0] = (const uint16_t*)s0;
   a.w[1] = (const uint8_t*)w1; a.s[1] = (const uint16_t*)s1;
   a.out = out; a.K = K; a.M = M; a.bs_shift = __builtin_ctz((unsigned)(bs / 32));
-  const dim3 grid((unsigned)((M + 15) / 16)), block(256);
-  const unsigned lds = (unsigned)K * 4;
+  const PageShape p = page_shape(M, K / 32);
   hipStream_t st = (hipStream_t)stream;
-  if (!in16 && out16 && ns == 1) hipLaunchKernelGGL((k_nvfp4_scalar<false, true, 1>), grid, block, lds, st, a);
-  else if (!in16 && !out16 && ns == 1) hipLaunchKernelGGL((k_nvfp4_scalar<false, false, 1>), grid, block, lds, st, a);
-  else if (in16 && out16 && ns == 1) hipLaunchKernelGGL((k_nvfp4_scalar<true, true, 1>), grid, block, lds, st, a);
-  else if (!in16 && out16 && ns == 2) hipLaunchKernelGGL((k_nvfp4_scalar<false, true, 2>), grid, block, lds, st, a);
-  else if (!in16 && !out16 && ns == 2) hipLaunchKernelGGL((k_nvfp4_scalar<false, false, 2>), grid, block, lds, st, a);
+#define VIB3_SCALAR_L(I, O, N, LL, ONE) \
+  hipLaunchKernelGGL((k_nvfp4_scalar_rows<I, O, N, LL, ONE>), dim3(p.grid), dim3(p.block), 0, st, a)
+#define VIB3_SCALAR(I, O, N)                          \
+  do {                                                \
+    if (p.L == 16) VIB3_SCALAR_L(I, O, N, 16, true);  \
+    else if (p.L == 32) VIB3_SCALAR_L(I, O, N, 32, true); \
+    else if (p.one) VIB3_SCALAR_L(I, O, N, 64, true); \
+    else VIB3_SCALAR_L(I, O, N, 64, false);           \
+  } while (0)
+  if (!in16 && out16 && ns == 1) VIB3_SCALAR(false, true, 1);
+  else if (!in16 && !out16 && ns == 1) VIB3_SCALAR(false, false, 1);
+  else if (in16 && out16 && ns == 1) VIB3_SCALAR(true, true, 1);
+  else if (!in16 && out16 && ns == 2) VIB3_SCALAR(false, true, 2);
+  else if (!in16 && !out16 && ns == 2) VIB3_SCALAR(false, false, 2);
   else return VIB3_ERR_UNSUPPORTED;
+#undef VIB3_SCALAR
+#undef VIB3_SCALAR_L
   VIB3_RETURN_LAUNCH();
 }
 
