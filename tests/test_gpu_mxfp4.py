@@ -227,3 +227,28 @@ def test_graph_replay_equals_eager():
         _say(f"  replay {r}")
         assert np.array_equal(got, want.view(torch.int16).cpu().numpy())
     del graph
+
+
+@pytest.mark.parametrize("hidden,inter,E,T,k", [(2048, 1024, 12, 360, 6), (2304, 1280, 10, 330, 6)])
+def test_wide_items_match_oracle(hidden, inter, E, T, k):
+    """Batches whose multi-block chunks run as wide items (64-token column blocks): whole 64-token
+    chunks, remainders of 17..63 tokens (wide) and 1..16 (narrow), an expert never picked and
+    out-of-range picks; k steps of 512 and of 256 only. Every token against the oracle; repeated
+    launches equal."""
+    _say(f"[mxfp4] wide hidden={hidden} inter={inter} E={E} T={T} k={k}")
+    from vib3_amd.mxfp4 import zipf_picks
+    bank = _bank(hidden, inter, E)
+    ids, w = zipf_picks(T, E - 1, k, s=0.9, seed=T)
+    ids[7, 2] = E + 3
+    rare = int(np.argmin(np.bincount(ids[ids < E].ravel(), minlength=E)[:E - 1]))
+    drop = np.flatnonzero((ids == rare).any(1))[64 + 9:]  # one chunk and a narrow remainder left
+    ids[drop] = np.where(ids[drop] == rare, E + 1, ids[drop])
+    counts = np.bincount(ids[ids < E].ravel(), minlength=E)
+    blocks = min(inter // 128, hidden // 256)
+    wide = int((counts // 64 + (counts % 64 > 16)).sum())
+    assert T * k // 64 * blocks > 256 and wide * blocks >= 256  # the launch rule for 256 CUs
+    assert counts[E - 1] == 0 and counts[rare] == 64 + 9
+    x, xh = _x(T, hidden, stream=79)
+    got = _run(bank, x, ids, w)
+    assert np.array_equal(got, _run(bank, x, ids, w))
+    _check(got, _oracle(bank, xh, ids, w))

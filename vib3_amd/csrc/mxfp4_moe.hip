@@ -50,7 +50,7 @@ struct MxArgs {
   const int* it_d;            // [items] distinct index of each work item
   const int* it_p0;           // [items] first entry of the item's token chunk within its expert
   const int* it_np;           // [items] token blocks of the chunk (1..4) | part << 8
-  const int* nitems;
+  const int* nitems;          // [2] narrow items, wide items (which follow them in the lists)
   const int* ent_tok;         // [T*top_k] token of each entry (grouped by expert)
   const int* ent_slot;        // [T*top_k] t*top_k + j of each entry
   const int* c_dix;           // [ncold] distinct index of each cold expert (row path): the
@@ -484,6 +484,187 @@ __global__ __launch_bounds__(64 * kMx2W) void k_mx_gemm2(MxArgs a) {
   }
 }
 
+// ------------------------------------------------------------------ matrix-core path, wide items
+//
+// Chunks of 17 to 64 tokens of one expert in one workgroup: the weights are read and decoded once
+// for up to four 16-token column blocks instead of once per block. Four waves, each with four 16-row
+// tiles (gate/up: two up tiles and the same two gate tiles, so SwiGLU stays in registers; down: four
+// row tiles) and NB column blocks, so one LDS read of a token fragment feeds four MFMAs and one
+// decoded weight fragment NB: per 32-wide slice and wave 16 NB matrix cycles per tile against 4 NB
+// LDS reads (half the LDS rate with all SIMDs busy) and 16 conversions. Steps are 256 wide: a lane's
+// two 16-byte pieces per row and step make whole 128-byte lines, and 64 tokens' activations take
+// 33 KB of LDS (one buffer: the next step's wait in registers), so two workgroups share a CU.
+// Eight experts with 512 tokens each at 4096 x 4096: 314 + 164 us = 0.87 PFLOP/s (980 -> 470 us per
+// batch); 512 tokens x top-8 over 384 experts (Zipf 1.1, Kimi shape) 1970 -> 1740 us. A second LDS
+// buffer (one barrier per step) measured 3 % slower, one workgroup per CU, which leaves registers
+// for the memory-bound kernels beside it, 3-20 % slower.
+constexpr int kMxWK = 256;             // k per step
+constexpr int kMxWPitch = kMxWK + 8;   // LDS row pitch (halves), against bank conflicts
+
+template <bool GATEUP, int NB>
+__device__ __forceinline__ void mx_wide(const MxArgs& a, int e, int o_e, int t_e, int p0,
+                                        uint16_t (&xs)[4 * kMxTokBlk][kMxWPitch]) {
+  const int tid = (int)threadIdx.x, lane = lane_id();
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rr = lane & 15, g = lane >> 4;
+  const int K = GATEUP ? a.hidden : a.inter;  // reduction
+  const int M = GATEUP ? a.inter : a.hidden;  // rows of each matrix
+  const int r0 = ((int)blockIdx.x * 4 + wave) * (GATEUP ? 32 : 64);
+  const size_t pkb = (size_t)K / 2, nsb = (size_t)K / 32;
+  const uint8_t* m0 = (const uint8_t*)a.table[(size_t)e * 3 + (GATEUP ? 0 : 2)];
+  const uint8_t* m1 = GATEUP ? (const uint8_t*)a.table[(size_t)e * 3 + 1] : m0;
+  const uint8_t* code[kMxTiles];
+  const uint8_t* scl[kMxTiles];
+#pragma unroll
+  for (int t = 0; t < kMxTiles; t++) {
+    const uint8_t* base = GATEUP ? (t < 2 ? m0 : m1) : m0;
+    const int row = GATEUP ? r0 + (t & 1) * 16 + rr : r0 + t * 16 + rr;
+    code[t] = base + (size_t)row * pkb + (size_t)g * 16;
+    scl[t] = base + (size_t)M * pkb + (size_t)row * nsb;
+  }
+  // activation staging: load i copies piece tid % 32 of token 8 i + tid / 32, whole 512-byte rows
+  // (a column past the expert's tokens repeats the chunk's first token and is never stored)
+  uint32_t xo[2 * NB];
+  const uint8_t* xb = (const uint8_t*)(GATEUP ? a.x : a.h);
+#pragma unroll
+  for (int i = 0; i < 2 * NB; i++) {
+    const int tok = p0 + 8 * i + (tid >> 5), tk = tok < t_e ? tok : p0;
+    const uint32_t rowi = (uint32_t)(GATEUP ? a.ent_tok[o_e + tk] : o_e + tk);
+    xo[i] = rowi * (uint32_t)(2 * K) + 16u * (uint32_t)(tid & 31);
+  }
+  struct W {
+    uint4 w[kMxTiles][2];
+    uint2 sc[kMxTiles];
+  };
+  auto load_w = [&](W& w, int k0) {
+#pragma unroll
+    for (int t = 0; t < kMxTiles; t++) {
+      w.w[t][0] = ld16(code[t] + k0 / 2);
+      w.w[t][1] = ld16(code[t] + k0 / 2 + 64);
+      w.sc[t] = ld8(scl[t] + k0 / 32);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  uint4 xv[2 * NB];
+  auto load_x = [&](int k0) {
+#pragma unroll
+    for (int i = 0; i < 2 * NB; i++) xv[i] = ld16(xb + xo[i] + 2u * (uint32_t)k0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto store_x = [&]() {
+#pragma unroll
+    for (int i = 0; i < 2 * NB; i++)
+      *(uint4*)&xs[8 * i + (tid >> 5)][(tid & 31) * 8] = xv[i];
+  };
+  f32x4_t acc[kMxTiles][NB];
+#pragma unroll
+  for (int t = 0; t < kMxTiles; t++)
+#pragma unroll
+    for (int b = 0; b < NB; b++) acc[t][b] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](const W& w) {
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        uint4 xf[NB];
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+          xf[b] = *(const uint4*)&xs[16 * b + rr][h * 128 + g * 32 + q * 8];
+#pragma unroll
+        for (int t = 0; t < kMxTiles; t++) {
+          // piece h of the step holds k = 128 h + 32 g ..: E8M0 byte 4 h + g
+          const float scale = e8m0_scale((uint8_t)((h ? w.sc[t].y : w.sc[t].x) >> (8 * g)));
+          const uint32_t words[4] = {w.w[t][h].x, w.w[t][h].y, w.w[t][h].z, w.w[t][h].w};
+          bf16x8_t ab;
+          f16x8_t ah;
+          decode8<GATEUP>(words[q], scale, ab, ah);
+#pragma unroll
+          for (int b = 0; b < NB; b++) {
+            if (GATEUP)
+              acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  ab, __builtin_bit_cast(bf16x8_t, xf[b]), acc[t][b], 0, 0, 0);
+            else
+              acc[t][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  ah, __builtin_bit_cast(f16x8_t, xf[b]), acc[t][b], 0, 0, 0);
+          }
+        }
+      }
+    }
+  };
+  // step s computes from W and LDS while step s + 1's activations and weights are on their way
+  // (activations first: waiting for them does not wait for the weights)
+  const int nsteps = K / kMxWK;
+  W A, B;
+  load_x(0);
+  load_w(A, 0);
+  store_x();
+  __syncthreads();
+  for (int s = 0;; s += 2) {
+    const int k1 = min(s + 1, nsteps - 1) * kMxWK, k2 = min(s + 2, nsteps - 1) * kMxWK;
+    load_x(k1);
+    load_w(B, k1);
+    compute(A);
+    if (s + 1 >= nsteps) break;
+    __syncthreads();
+    store_x();
+    __syncthreads();
+    load_x(k2);
+    load_w(A, k2);
+    compute(B);
+    if (s + 2 >= nsteps) break;
+    __syncthreads();
+    store_x();
+    __syncthreads();
+  }
+  // epilogue: lane holds rows g * 4 + i of each tile for token column rr of each block
+#pragma unroll
+  for (int b = 0; b < NB; b++) {
+    const int tok = p0 + 16 * b + rr;
+    if (tok >= t_e) continue;
+    if (GATEUP) {
+#pragma unroll
+      for (int half = 0; half < 2; half++) {
+        uint16_t hv[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          const float up = acc[half][b][i], gate = acc[2 + half][b][i];
+          hv[i] = f32_to_f16_bits((gate / (1.0f + expf(-gate))) * up);  // kernels.rs:3041
+        }
+        *(uint2*)(a.h + (size_t)(o_e + tok) * M + r0 + half * 16 + g * 4) =
+            make_uint2((uint32_t)hv[0] | ((uint32_t)hv[1] << 16),
+                       (uint32_t)hv[2] | ((uint32_t)hv[3] << 16));
+      }
+    } else {
+      const int slot = a.ent_slot[o_e + tok];
+#pragma unroll
+      for (int t = 0; t < kMxTiles; t++) {
+        uint16_t dv[4];
+#pragma unroll
+        for (int i = 0; i < 4; i++) dv[i] = f32_to_f16_bits(acc[t][b][i]);
+        *(uint2*)(a.d + (size_t)slot * M + r0 + t * 16 + g * 4) =
+            make_uint2((uint32_t)dv[0] | ((uint32_t)dv[1] << 16),
+                       (uint32_t)dv[2] | ((uint32_t)dv[3] << 16));
+      }
+    }
+  }
+}
+
+// blockIdx.y = wide item (listed after the narrow ones), blockIdx.x = block of 128 gate/up row pairs
+// or 256 down rows.
+template <bool GATEUP>
+__global__ __launch_bounds__(256, 2) void k_mx_wide(MxArgs a) {
+  __shared__ __attribute__((aligned(16))) uint16_t xs[4 * kMxTokBlk][kMxWPitch];
+  if ((int)blockIdx.y >= a.nitems[1]) return;
+  const int item = a.nitems[0] + (int)blockIdx.y;
+  const int dix = a.it_d[item];
+  const int e = a.d_expert[dix], o_e = a.d_off[dix], t_e = a.d_cnt[dix];
+  const int p0 = a.it_p0[item], nb = a.it_np[item];
+  if (nb == 4) mx_wide<GATEUP, 4>(a, e, o_e, t_e, p0, xs);
+  else if (nb == 3) mx_wide<GATEUP, 3>(a, e, o_e, t_e, p0, xs);
+  else if (nb == 2) mx_wide<GATEUP, 2>(a, e, o_e, t_e, p0, xs);
+  else mx_wide<GATEUP, 1>(a, e, o_e, t_e, p0, xs);
+}
+
 // ----------------------------------------------------------------------------- row path
 //
 // Experts picked by at most kMxColdMax tokens (three quarters of the touched experts of a
@@ -660,9 +841,20 @@ __host__ __device__ constexpr int mx_chunk_blocks(int c) { return (c + kMxTokBlk
 
 // Work items of an expert with c entries: one per part of each 64-token chunk.
 __host__ __device__ inline int mx_expert_items(int c) {
-  int n = 0;
-  for (int p0 = 0; p0 < c; p0 += kMxChunk) n += mx_chunk_blocks(c - p0 < kMxChunk ? c - p0 : kMxChunk);
-  return n;
+  return c / kMxChunk * (kMxChunk / kMxTokBlk) + mx_chunk_blocks(c % kMxChunk);
+}
+
+// With wide items: chunks of more than one block are one wide item each, the last chunk's single
+// block (1..16 tokens) a narrow one. Which of an expert's tokens that block holds is not fixed, so
+// both kinds must form the same sums: k_mx_gemm2, k_mx_gemm<false, 1> and k_mx_wide all run k in
+// order, k_mx_gemm<true, 4> (hidden no multiple of k_mx_gemm2's step) does not. There (`all`) every
+// chunk of an expert with more than one block is wide.
+__host__ __device__ inline int mx_expert_wide(int c, bool all) {
+  return c / kMxChunk + (c % kMxChunk > (all && c > kMxTokBlk ? 0 : kMxTokBlk));
+}
+__host__ __device__ inline int mx_expert_narrow(int c, bool all) {
+  const int r = c % kMxChunk;
+  return r > 0 && r <= kMxTokBlk && !(all && c > kMxTokBlk);
 }
 
 // Group the T*top_k picks by expert (one workgroup). An expert's entries sit in the order its
@@ -686,12 +878,14 @@ struct MxGroupArgs {
   int* ncold;           // experts first)
   int* ncold1;
   int top_k;
+  int wide_min;         // with at least so many multi-block chunks (> 0) they are wide items, listed
+                        // after the narrow ones; else 16-token narrow items
+  int wide_all;         // (see mx_expert_wide)
 };
 
 __global__ __launch_bounds__(1024) void k_mx_group(MxGroupArgs a) {
   __shared__ int cnt[kMaxExperts];
   __shared__ int off[kMaxExperts];
-  __shared__ int part[1024], dpart[1024], ipart[1024], cpart[1024];
   static_assert(kMxColdMax == 2, "the row path lists one- and two-token experts");
   __shared__ __attribute__((aligned(16))) uint16_t sid[kMxMaxPicks];
   const int tid = (int)threadIdx.x, nt = (int)blockDim.x;
@@ -714,18 +908,24 @@ __global__ __launch_bounds__(1024) void k_mx_group(MxGroupArgs a) {
   const int e0 = min(a.E, tid * span), e1 = min(a.E, e0 + span);
   // experts with 1..kMxColdMax entries go to the row path, the others to matrix-core items
   // row-path experts are listed one-token ones first, then two-token ones (one launch each)
-  int s = 0, ds = 0, is = 0, c1 = 0, c2 = 0;
+  int s = 0, ds = 0, is = 0, c1 = 0, c2 = 0, ws = 0, ns = 0;
   for (int e = e0; e < e1; e++) {
     s += cnt[e];
     ds += cnt[e] > 0;
-    is += cnt[e] > kMxColdMax ? mx_expert_items(cnt[e]) : 0;
+    if (cnt[e] > kMxColdMax) {
+      is += mx_expert_items(cnt[e]);
+      ns += mx_expert_narrow(cnt[e], a.wide_all);
+      ws += mx_expert_wide(cnt[e], a.wide_all);
+    }
     c1 += cnt[e] == 1;
     c2 += cnt[e] == 2;
   }
-  // inclusive scans of the five counts over the workgroup: within each wave by lane shuffles,
-  // then over the (at most 16) wave totals, with two barriers in all
-  constexpr int kQ = 5;
-  int sc[kQ] = {s, ds, is, c1, c2};
+  // Inclusive scans of the counts over the workgroup: within each wave by lane shuffles, then over
+  // the wave totals, which every thread adds up itself (independent reads, one barrier). Counts are
+  // at most kMxMaxPicks, so two share a word.
+  constexpr int kQ = 4;
+  static_assert(kMxMaxPicks < 1 << 15, "two counts to a word");
+  int sc[kQ] = {s | ds << 16, is | c1 << 16, c2 | ws << 16, ns};
   const int lane = tid & 63, wv = tid >> 6;
 #pragma unroll
   for (int st = 1; st < 64; st <<= 1) {
@@ -735,31 +935,31 @@ __global__ __launch_bounds__(1024) void k_mx_group(MxGroupArgs a) {
       if (lane >= st) sc[q] += v;
     }
   }
-  __shared__ int wtot[16][kQ];
-  __shared__ int tot[kQ];
+  __shared__ __attribute__((aligned(16))) int wtot[16][kQ];
   if (lane == 63) {
 #pragma unroll
     for (int q = 0; q < kQ; q++) wtot[wv][q] = sc[q];
   }
   __syncthreads();
-  if (tid < kQ) {  // thread q scans the wave totals of count q
-    int acc = 0;
-    for (int w = 0; w < nt / 64; w++) {
-      const int v = wtot[w][tid];
-      wtot[w][tid] = acc;  // exclusive: what the waves before w hold
-      acc += v;
-    }
-    tot[tid] = acc;
-  }
-  __syncthreads();
+  int tot[kQ] = {0, 0, 0, 0};
 #pragma unroll
-  for (int q = 0; q < kQ; q++) sc[q] += wtot[wv][q];
-  part[tid] = sc[0];
-  dpart[tid] = sc[1];
-  ipart[tid] = sc[2];
-  cpart[tid] = tot[3] + tot[4];
-  int run = part[tid] - s, drun = dpart[tid] - ds, irun = ipart[tid] - is;
-  int c1run = sc[3] - c1, c2run = tot[3] + sc[4] - c2;
+  for (int w = 0; w < 16; w++) {  // (the launch has 16 waves)
+#pragma unroll
+    for (int q = 0; q < kQ; q++) {
+      const int v = wtot[w][q];
+      if (w < wv) sc[q] += v;
+      tot[q] += v;
+    }
+  }
+  auto lo = [](int v) { return v & 0xffff; };
+  auto hi = [](int v) { return v >> 16; };
+  const int ncold1 = hi(tot[1]), ncold2 = lo(tot[2]);
+  const bool wide = a.wide_min > 0 && hi(tot[2]) >= a.wide_min;
+  if (wide) is = ns;  // the narrow items are the last chunks' single blocks only
+  const int nitems = wide ? tot[3] : lo(tot[1]);
+  int run = lo(sc[0]) - s, drun = hi(sc[0]) - ds, irun = (wide ? sc[3] : lo(sc[1])) - is;
+  int c1run = hi(sc[1]) - c1, c2run = ncold1 + lo(sc[2]) - c2;
+  int wrun = nitems + hi(sc[2]) - ws;  // wide items follow the narrow ones
   for (int e = e0; e < e1; e++) {
     off[e] = run;
     if (cnt[e] == 1) a.c_dix[c1run++] = drun;
@@ -770,6 +970,13 @@ __global__ __launch_bounds__(1024) void k_mx_group(MxGroupArgs a) {
       a.d_cnt[drun] = cnt[e];
       for (int p0 = 0; cnt[e] > kMxColdMax && p0 < cnt[e]; p0 += kMxChunk) {
         const int nb = mx_chunk_blocks(min(kMxChunk, cnt[e] - p0));
+        if (wide && (nb > 1 || (a.wide_all && cnt[e] > kMxTokBlk))) {
+          a.it_d[wrun] = drun;
+          a.it_p0[wrun] = p0;
+          a.it_np[wrun] = nb;
+          wrun++;
+          continue;
+        }
         for (int part = 0; part < nb; part++) {
           a.it_d[irun] = drun;
           a.it_p0[irun] = p0;
@@ -782,10 +989,11 @@ __global__ __launch_bounds__(1024) void k_mx_group(MxGroupArgs a) {
     run += cnt[e];
   }
   if (tid == nt - 1) {
-    *a.nd = dpart[nt - 1];
-    *a.nitems = ipart[nt - 1];
-    *a.ncold = tot[3] + tot[4];
-    *a.ncold1 = tot[3];
+    *a.nd = hi(tot[0]);
+    a.nitems[0] = nitems;
+    a.nitems[1] = wide ? hi(tot[2]) : 0;
+    *a.ncold = ncold1 + ncold2;
+    *a.ncold1 = ncold1;
   }
 
   __syncthreads();
@@ -888,7 +1096,8 @@ static void mx_launch_rows(const MxArgs& a, int K, hipStream_t st1, hipStream_t 
 // device); under graph capture the fork and join become graph edges.
 struct MxSide {
   hipStream_t st = nullptr, st2 = nullptr;  // one-token and two-token row paths
-  hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr;
+  hipStream_t st3 = nullptr;                // wide items
+  hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr, join3 = nullptr;
   bool ok = false;
 };
 #ifndef VIB3_MX_THREE_STREAMS
@@ -908,11 +1117,13 @@ static MxSide* mx_side() {  // called with the lock held
   MxSide& s = g_mx_side[dev];
   if (!s.ok) {
     if (hipStreamCreateWithFlags(&s.st, hipStreamNonBlocking) != hipSuccess ||
-        hipStreamCreateWithFlags(&s.st2, hipStreamNonBlocking) != hipSuccess)
+        hipStreamCreateWithFlags(&s.st2, hipStreamNonBlocking) != hipSuccess ||
+        hipStreamCreateWithFlags(&s.st3, hipStreamNonBlocking) != hipSuccess)
       return nullptr;
     if (hipEventCreateWithFlags(&s.fork, kMxEventFlags) != hipSuccess ||
         hipEventCreateWithFlags(&s.join, kMxEventFlags) != hipSuccess ||
-        hipEventCreateWithFlags(&s.join2, kMxEventFlags) != hipSuccess)
+        hipEventCreateWithFlags(&s.join2, kMxEventFlags) != hipSuccess ||
+        hipEventCreateWithFlags(&s.join3, kMxEventFlags) != hipSuccess)
       return nullptr;
     s.ok = true;
   }
@@ -944,6 +1155,23 @@ static int mx_grid_items(const vib3_moe_mxfp4_batch* B) {
   return bound < cap ? bound : cap;
 }
 
+// Wide items: the most a batch can form (every expert's but its last has 64 tokens, and an expert with
+// any has more than kMxTokBlk: the launches' grid rows) and the fewest for which k_mx_group lists them: the smaller of the two phases' grids then
+// gives every CU a workgroup. With fewer, 16-token blocks win, as they spread over more CUs (18
+// experts, 67 tokens x top-2 at 2560 x 1792: 81 us narrow, 106 us wide; 16 experts, 489 tokens x
+// top-2 at 5376 x 4096: 590 us narrow, 277 us wide). The counts are only known on the device, and
+// launches that find no wide item still cost 12 us of a 655 us batch (64 tokens x top-8, Kimi
+// shape), so they are left out unless the picks alone make more than a CU's worth of 64-token items.
+struct MxWide {
+  int min, max;
+};
+static MxWide mx_wide_items(const vib3_moe_mxfp4_batch* B) {
+  const int n = B->tokens * B->top_k;
+  const int gu = B->inter / 128, dn = B->hidden / 256, blocks = gu < dn ? gu : dn;
+  if (n / kMxChunk * blocks <= device_cus()) return MxWide{0, 0};
+  return MxWide{(device_cus() + blocks - 1) / blocks, n / (kMxTokBlk + 1)};
+}
+
 static MxWs mx_ws(const vib3_moe_mxfp4_batch* B) {
   MxWs w{};
   const size_t n = (size_t)B->tokens * B->top_k;
@@ -960,7 +1188,7 @@ static MxWs mx_ws(const vib3_moe_mxfp4_batch* B) {
   w.it_d = take(sizeof(int) * (size_t)mx_max_items(B));
   w.it_p0 = take(sizeof(int) * (size_t)mx_max_items(B));
   w.it_np = take(sizeof(int) * (size_t)mx_max_items(B));
-  w.nitems = take(sizeof(int));
+  w.nitems = take(2 * sizeof(int));
   w.ent_tok = take(sizeof(int) * n);
   w.ent_slot = take(sizeof(int) * n);
   w.c_dix = take(sizeof(int) * B->num_experts);
@@ -1011,6 +1239,9 @@ int vib3_launch_moe_mxfp4_batched(const vib3_moe_mxfp4_batch* B, void* stream) {
   ga.c_dix = (int*)(ws + w.c_dix); ga.ncold = (int*)(ws + w.ncold);
   ga.ncold1 = (int*)(ws + w.ncold1);
   ga.top_k = B->top_k;
+  const MxWide wide = mx_wide_items(B);
+  ga.wide_min = wide.min;
+  ga.wide_all = B->hidden % kMx2K != 0;
   hipLaunchKernelGGL(k_mx_group, dim3(1), dim3(1024), 0, st, ga);
 
   MxArgs a{};
@@ -1031,14 +1262,22 @@ int vib3_launch_moe_mxfp4_batched(const vib3_moe_mxfp4_batch* B, void* stream) {
     lock.lock();
     side = mx_side();
   }
-  hipStream_t rs = st, rs2 = st;  // the row paths' streams
+  hipStream_t rs = st, rs2 = st, ws3 = st;  // the streams of the row paths and the wide items
   if (side) {
     hipError_t e = hipEventRecord(side->fork, st);
     if (e == hipSuccess) e = hipStreamWaitEvent(side->st, side->fork, 0);
     if (e == hipSuccess && kMxThreeStreams) e = hipStreamWaitEvent(side->st2, side->fork, 0);
+    if (e == hipSuccess && wide.max > 0) e = hipStreamWaitEvent(side->st3, side->fork, 0);
     if (e != hipSuccess) return (int)e;
+    ws3 = side->st3;
     rs = side->st;
     rs2 = kMxThreeStreams ? side->st2 : side->st;
+  }
+  if (wide.max > 0) {
+    hipLaunchKernelGGL((k_mx_wide<true>), dim3((unsigned)(B->inter / 128), (unsigned)wide.max),
+                       dim3(256), 0, ws3, a);
+    hipLaunchKernelGGL((k_mx_wide<false>), dim3((unsigned)(B->hidden / 256), (unsigned)wide.max),
+                       dim3(256), 0, ws3, a);
   }
   mx_launch_rows<true>(a, B->hidden, rs, rs2);
   mx_launch_rows<false>(a, B->inter, rs, rs2);
@@ -1065,6 +1304,8 @@ int vib3_launch_moe_mxfp4_batched(const vib3_moe_mxfp4_batch* B, void* stream) {
     if (e == hipSuccess) e = hipStreamWaitEvent(st, side->join, 0);
     if (e == hipSuccess && kMxThreeStreams) e = hipEventRecord(side->join2, rs2);
     if (e == hipSuccess && kMxThreeStreams) e = hipStreamWaitEvent(st, side->join2, 0);
+    if (e == hipSuccess && wide.max > 0) e = hipEventRecord(side->join3, ws3);
+    if (e == hipSuccess && wide.max > 0) e = hipStreamWaitEvent(st, side->join3, 0);
     if (e != hipSuccess) return (int)e;
   }
   hipLaunchKernelGGL(k_mx_combine, dim3((unsigned)((B->hidden + 2047) / 2048), (unsigned)B->tokens),
