@@ -812,14 +812,15 @@ __device__ __forceinline__ void mx_rows_segment(const MxArgs& a, int e, int o_e,
   }
 }
 
-// One launch per token count: the one-token experts' segments hold half the activation
-// registers of the two-token ones, so their kernel keeps more waves per SIMD.
+// NT = 1 / 2: one launch per token count (the one-token experts' segments hold half the activation
+// registers of the two-token ones, so their kernel keeps more waves per SIMD). NT = 0: both in one
+// launch (small batches, see the launcher).
 template <bool GATEUP, int NCH, int NT>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NT == 1 && (GATEUP || NCH <= 2) ? 3 : 1)))
 void k_mx_rows(MxArgs a) {
-  const int n1 = *a.ncold1;
-  const int first = NT == 1 ? 0 : n1;
-  const int ncold = NT == 1 ? n1 : *a.ncold - n1;
+  const int n1 = *a.ncold1, n12 = *a.ncold;
+  const int first = NT == 2 ? n1 : 0;
+  const int ncold = NT == 0 ? n12 : NT == 1 ? n1 : n12 - n1;
   const int per = GATEUP ? a.inter : a.hidden / 4;  // items per expert
   const long n = (long)ncold * per;
   const int W = (int)gridDim.x * 4;
@@ -831,7 +832,8 @@ void k_mx_rows(MxArgs a) {
     const int q1 = (int)min((long)per, i1 - (long)c * per);
     const int dix = a.c_dix[first + c];
     const int e = a.d_expert[dix], o_e = a.d_off[dix];
-    mx_rows_segment<GATEUP, NCH, NT>(a, e, o_e, q0, q1);
+    if (NT == 1 || (NT == 0 && c < n1)) mx_rows_segment<GATEUP, NCH, 1>(a, e, o_e, q0, q1);
+    else mx_rows_segment<GATEUP, NCH, 2>(a, e, o_e, q0, q1);
     i = (long)c * per + q1;
   }
 }
@@ -1076,34 +1078,35 @@ static void mx_launch_rows_one(const MxArgs& a, hipStream_t st) {
   hipLaunchKernelGGL((k_mx_rows<GATEUP, NCH, NT>), dim3((unsigned)g), dim3(256), 0, st, a);
 }
 
-// Row-path launches (one-token and two-token experts): K = the reduction length picks the
-// chunks per lane (K <= 8192).
+// Row-path launches (one-token and two-token experts, or both in one launch): K = the reduction
+// length picks the chunks per lane (K <= 8192).
+template <bool GATEUP, int NCH>
+static void mx_launch_rows_n(const MxArgs& a, bool merged, hipStream_t st1, hipStream_t st2) {
+  if (merged) return mx_launch_rows_one<GATEUP, NCH, 0>(a, st1);
+  mx_launch_rows_one<GATEUP, NCH, 1>(a, st1);
+  mx_launch_rows_one<GATEUP, NCH, 2>(a, st2);
+}
 template <bool GATEUP>
-static void mx_launch_rows(const MxArgs& a, int K, hipStream_t st1, hipStream_t st2) {
+static void mx_launch_rows(const MxArgs& a, int K, bool merged, hipStream_t st1, hipStream_t st2) {
   switch ((K / 32 + 63) / 64) {
-    case 1: mx_launch_rows_one<GATEUP, 1, 1>(a, st1); mx_launch_rows_one<GATEUP, 1, 2>(a, st2); break;
-    case 2: mx_launch_rows_one<GATEUP, 2, 1>(a, st1); mx_launch_rows_one<GATEUP, 2, 2>(a, st2); break;
-    case 3: mx_launch_rows_one<GATEUP, 3, 1>(a, st1); mx_launch_rows_one<GATEUP, 3, 2>(a, st2); break;
-    default: mx_launch_rows_one<GATEUP, 4, 1>(a, st1); mx_launch_rows_one<GATEUP, 4, 2>(a, st2); break;
+    case 1: return mx_launch_rows_n<GATEUP, 1>(a, merged, st1, st2);
+    case 2: return mx_launch_rows_n<GATEUP, 2>(a, merged, st1, st2);
+    case 3: return mx_launch_rows_n<GATEUP, 3>(a, merged, st1, st2);
+    default: return mx_launch_rows_n<GATEUP, 4>(a, merged, st1, st2);
   }
 }
 
-// The two paths are independent until the combine: the matrix-core launches (hot experts) run
-// on the caller's stream and the row-path launches (cold experts) on a second stream of the
-// library (one per device, default priority), forked after the grouping and joined before the
-// combine with events, so each path fills the other's ramps and tails. Enqueueing is
-// serialised by a lock (the side stream and its two events are shared by every call on that
-// device); under graph capture the fork and join become graph edges.
+// The paths are independent until the combine. Larger batches run them on streams of the library
+// beside the caller's (three per device, default priority), forked after the grouping and joined
+// before the combine with events, so each path fills the others' ramps and tails (mx_streams says
+// when). Enqueueing is serialised by a lock (the side streams and their events are shared by every
+// call on that device); under graph capture the fork and join become graph edges.
 struct MxSide {
   hipStream_t st = nullptr, st2 = nullptr;  // one-token and two-token row paths
   hipStream_t st3 = nullptr;                // wide items
   hipEvent_t fork = nullptr, join = nullptr, join2 = nullptr, join3 = nullptr;
   bool ok = false;
 };
-#ifndef VIB3_MX_THREE_STREAMS
-#define VIB3_MX_THREE_STREAMS 1  // (build-time switch: the two row paths on streams of their own)
-#endif
-constexpr bool kMxThreeStreams = VIB3_MX_THREE_STREAMS;
 // The fork and join events order work of one device only: device-scope fences suffice, and
 // skipping the system-scope ones (cache write-back and invalidation at each event) took ~4.5 us
 // off a c4 batch.
@@ -1153,6 +1156,24 @@ static int mx_grid_items(const vib3_moe_mxfp4_batch* B) {
   const int bound = (n + (kMxTokBlk - 1) * m) / kMxTokBlk;
   const int cap = mx_max_items(B);
   return bound < cap ? bound : cap;
+}
+
+// How a batch's chains run (us per batch, one stream / two / four; Kimi shape unless said):
+//   * one: everything on the caller's stream, the row paths in one launch per phase. The fork and the
+//     joins cost the host 30 us and the GPU several, which few picks or small experts do not win back:
+//     1 token x top-8 51 / 56 / 84, 2 tokens 77 / 82 / 107, 4 tokens of 128 experts of 2048 x 768
+//     35 / 55 / 81.
+//   * two: the matrix-core chain beside the row paths (one launch per phase). 4 tokens 140 / 118 /
+//     136, 16 tokens 317 / 300 / 314, 32 tokens 468 / 438 / 447, of 2048 x 768 16 tokens 78 / 71 / 86
+//     and 64 tokens 103 / 102 / 109.
+//   * four: each row path and the wide items on streams of their own too, which pays once the
+//     one-token experts alone fill the GPU. 64 tokens 688 / 653 / 649, 128 tokens 1003 / 994 / 968.
+enum MxStreams { kMxOne, kMxTwo, kMxFour };
+static MxStreams mx_streams(const vib3_moe_mxfp4_batch* B) {
+  const int n = B->tokens * B->top_k;
+  const double bytes = 3.0 * (17.0 / 32) * B->hidden * B->inter * (n < B->num_experts ? n : B->num_experts);
+  if (n <= 16 || bytes < 200e6) return kMxOne;  // (weights of at most so many distinct experts)
+  return n <= 256 || bytes < 1e9 ? kMxTwo : kMxFour;
 }
 
 // Wide items: the most a batch can form (every expert's but its last has 64 tokens, and an expert with
@@ -1253,58 +1274,73 @@ int vib3_launch_moe_mxfp4_batched(const vib3_moe_mxfp4_batch* B, void* stream) {
   a.h = (uint16_t*)(ws + w.h); a.d = (uint16_t*)(ws + w.d);
   a.hidden = B->hidden; a.inter = B->inter;
   const unsigned items = (unsigned)mx_grid_items(B);
-  std::unique_lock<std::mutex> lock(g_mx_side_lock, std::defer_lock);
-  MxSide* side = nullptr;
-#ifndef VIB3_MX_ONE_STREAM
-#define VIB3_MX_ONE_STREAM 0  // (profiling builds: 1 = the three chains on the caller's stream)
-#endif
-  if (!VIB3_MX_ONE_STREAM) {
-    lock.lock();
-    side = mx_side();
-  }
-  hipStream_t rs = st, rs2 = st, ws3 = st;  // the streams of the row paths and the wide items
-  if (side) {
-    hipError_t e = hipEventRecord(side->fork, st);
-    if (e == hipSuccess) e = hipStreamWaitEvent(side->st, side->fork, 0);
-    if (e == hipSuccess && kMxThreeStreams) e = hipStreamWaitEvent(side->st2, side->fork, 0);
-    if (e == hipSuccess && wide.max > 0) e = hipStreamWaitEvent(side->st3, side->fork, 0);
-    if (e != hipSuccess) return (int)e;
-    ws3 = side->st3;
-    rs = side->st;
-    rs2 = kMxThreeStreams ? side->st2 : side->st;
-  }
-  if (wide.max > 0) {
-    hipLaunchKernelGGL((k_mx_wide<true>), dim3((unsigned)(B->inter / 128), (unsigned)wide.max),
-                       dim3(256), 0, ws3, a);
-    hipLaunchKernelGGL((k_mx_wide<false>), dim3((unsigned)(B->hidden / 256), (unsigned)wide.max),
-                       dim3(256), 0, ws3, a);
-  }
-  mx_launch_rows<true>(a, B->hidden, rs, rs2);
-  mx_launch_rows<false>(a, B->inter, rs, rs2);
   // matrix-core path: activations staged in LDS when k is a multiple of the step, otherwise
   // registers-only with k split over the waves (gate/up) or whole (down)
-  if (items == 0) {  // (no expert can take the matrix-core path)
-  } else if (B->hidden % kMx2K == 0)
-    hipLaunchKernelGGL((k_mx_gemm2<true, kMx2K>), dim3((unsigned)(B->inter / (16 * kMx2H)), items),
-                       dim3(64 * kMx2W), 0,
-                       st, a);
-  else
-    hipLaunchKernelGGL((k_mx_gemm<true, 4>), dim3((unsigned)(B->inter / 32), items), dim3(256), 0,
-                       st, a);
-  if (items == 0) {
-  } else if (B->inter % kMx2KD == 0)
-    hipLaunchKernelGGL((k_mx_gemm2<false, kMx2KD>), dim3((unsigned)(B->hidden / (16 * kMx2W)), items),
-                       dim3(64 * kMx2W),
-                       0, st, a);
-  else
-    hipLaunchKernelGGL((k_mx_gemm<false, 1>), dim3((unsigned)(B->hidden / 256), items), dim3(256),
-                       0, st, a);
-  if (side) {
-    hipError_t e = hipEventRecord(side->join, rs);
+  auto matrix_gateup = [&](hipStream_t q) {
+    if (items == 0) return;  // (no expert can take the matrix-core path)
+    if (B->hidden % kMx2K == 0)
+      hipLaunchKernelGGL((k_mx_gemm2<true, kMx2K>), dim3((unsigned)(B->inter / (16 * kMx2H)), items),
+                         dim3(64 * kMx2W), 0, q, a);
+    else
+      hipLaunchKernelGGL((k_mx_gemm<true, 4>), dim3((unsigned)(B->inter / 32), items), dim3(256), 0, q, a);
+  };
+  auto matrix_down = [&](hipStream_t q) {
+    if (items == 0) return;
+    if (B->inter % kMx2KD == 0)
+      hipLaunchKernelGGL((k_mx_gemm2<false, kMx2KD>), dim3((unsigned)(B->hidden / (16 * kMx2W)), items),
+                         dim3(64 * kMx2W), 0, q, a);
+    else
+      hipLaunchKernelGGL((k_mx_gemm<false, 1>), dim3((unsigned)(B->hidden / 256), items), dim3(256), 0, q, a);
+  };
+  auto wide_items = [&](hipStream_t q) {
+    if (wide.max == 0) return;
+    hipLaunchKernelGGL((k_mx_wide<true>), dim3((unsigned)(B->inter / 128), (unsigned)wide.max),
+                       dim3(256), 0, q, a);
+    hipLaunchKernelGGL((k_mx_wide<false>), dim3((unsigned)(B->hidden / 256), (unsigned)wide.max),
+                       dim3(256), 0, q, a);
+  };
+  const MxStreams mode = wide.max > 0 ? kMxFour : mx_streams(B);
+  std::unique_lock<std::mutex> lock(g_mx_side_lock, std::defer_lock);
+  MxSide* side = nullptr;
+  if (mode != kMxOne) {
+    lock.lock();
+    side = mx_side();
+    if (!side) lock.unlock();
+  }
+  hipError_t e = hipSuccess;
+  if (!side) {  // one stream
+    wide_items(st);
+    mx_launch_rows<true>(a, B->hidden, true, st, st);
+    matrix_gateup(st);
+    mx_launch_rows<false>(a, B->inter, true, st, st);
+    matrix_down(st);
+  } else if (mode == kMxTwo) {
+    e = hipEventRecord(side->fork, st);
+    mx_launch_rows<true>(a, B->hidden, true, st, st);
+    if (e == hipSuccess) e = hipStreamWaitEvent(side->st, side->fork, 0);
+    if (e != hipSuccess) return (int)e;
+    matrix_gateup(side->st);
+    mx_launch_rows<false>(a, B->inter, true, st, st);
+    matrix_down(side->st);
+    e = hipEventRecord(side->join, side->st);
     if (e == hipSuccess) e = hipStreamWaitEvent(st, side->join, 0);
-    if (e == hipSuccess && kMxThreeStreams) e = hipEventRecord(side->join2, rs2);
-    if (e == hipSuccess && kMxThreeStreams) e = hipStreamWaitEvent(st, side->join2, 0);
-    if (e == hipSuccess && wide.max > 0) e = hipEventRecord(side->join3, ws3);
+    if (e != hipSuccess) return (int)e;
+  } else {
+    e = hipEventRecord(side->fork, st);
+    if (e == hipSuccess) e = hipStreamWaitEvent(side->st, side->fork, 0);
+    if (e == hipSuccess) e = hipStreamWaitEvent(side->st2, side->fork, 0);
+    if (e == hipSuccess && wide.max > 0) e = hipStreamWaitEvent(side->st3, side->fork, 0);
+    if (e != hipSuccess) return (int)e;
+    wide_items(side->st3);
+    mx_launch_rows<true>(a, B->hidden, false, side->st, side->st2);
+    mx_launch_rows<false>(a, B->inter, false, side->st, side->st2);
+    matrix_gateup(st);
+    matrix_down(st);
+    e = hipEventRecord(side->join, side->st);
+    if (e == hipSuccess) e = hipStreamWaitEvent(st, side->join, 0);
+    if (e == hipSuccess) e = hipEventRecord(side->join2, side->st2);
+    if (e == hipSuccess) e = hipStreamWaitEvent(st, side->join2, 0);
+    if (e == hipSuccess && wide.max > 0) e = hipEventRecord(side->join3, side->st3);
     if (e == hipSuccess && wide.max > 0) e = hipStreamWaitEvent(st, side->join3, 0);
     if (e != hipSuccess) return (int)e;
   }
