@@ -1,0 +1,49 @@
+"""One INT4 page with k > 8192 and f16 activations: the staged-activation kernel (one chunk past four
+per lane, no multiple of a pass, the longest k its LDS holds, one to four rows per wave, few rows), and
+the shapes just outside it (scales not behind the rows, k past its LDS) that keep the split kernel."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+
+
+@pytest.mark.parametrize("k,m,g,sdt,apart", [
+    (8224, 1, 32, O.BF16, False), (8224, 523, 64, O.F16, False), (9216, 3073, 32, O.BF16, False),
+    (14336, 6149, 128, O.F16, False), (30816, 5, 32, O.BF16, False), (30848, 5, 32, O.BF16, False),
+    (8224, 37, 32, O.F16, True)])
+def test_long_k(k, m, g, sdt, apart):
+    from vib3_amd import _lib
+    print(f"case: long k={k} m={m} g={g} sdt={sdt} apart={apart}", flush=True)
+    x = O.synth_normal_array(7, 300 + k, 0, k, 1.0, O.F16)
+    page = O.synth_int4_page(0x5EED0000, 4000 + k, k, g, sdt, 0.02, 0, m)
+    xd = O.to_f32(x, O.F16).astype(np.float64)
+    b = page[:m * k // 2].reshape(m, k // 2)
+    q = np.stack([b & 15, b >> 4], 2).reshape(m, k).astype(np.float64) - 8
+    s = O.to_f32(page[m * k // 2:].view(np.uint16), sdt).astype(np.float64).reshape(m, -(-k // g)).repeat(g, 1)[:, :k]
+    ref = (q * s) @ xd
+    # f32: a term passes at most 40 roundings (16 of its chunk, 16 of its lane's chunks and passes, 8 of
+    # the reduction and scale), each 2^-24 of a partial sum no larger than the sum of |x| (|q - 8| + 8) s
+    # (the offset 8 is subtracted per chunk)
+    bound = 40 * 2.0 ** -24 * (((np.abs(q) + 8) * s) @ np.abs(xd))
+    dx, dp = torch.from_numpy(x.view(np.int16)).cuda(), torch.from_numpy(page).cuda()
+    st = torch.cuda.current_stream().cuda_stream
+    out = torch.full((m + 8,), 7.5, dtype=torch.float32, device="cuda")
+    out16 = torch.full((m + 8,), 7.5, dtype=torch.float16, device="cuda")
+    if apart:  # f16 scales in a buffer of their own: the reference's launcher, f16 out only
+        sc = dp[m * k // 2:].clone()
+        _lib.call("vib3_launch_partial_matmul_int4", dx.data_ptr(), dp.data_ptr(), sc.data_ptr(), out16.data_ptr(),
+                  k, m, g, st)
+    else:
+        for o, dt in ((out, _lib.DT_F32), (out16, _lib.DT_F16)):
+            _lib.call("vib3_launch_partial_matmul_int4_ex", dx.data_ptr(), O.F16, dp.data_ptr(), o.data_ptr(), dt, k,
+                      m, g, sdt, st)
+    torch.cuda.synchronize()
+    o, o16 = out.cpu().numpy(), out16.cpu().numpy()
+    assert (o[m:] == 7.5).all() and (o16[m:] == 7.5).all()
+    if not apart:
+        assert np.all(np.abs(o[:m] - ref) <= bound)
+        assert np.array_equal(o16[:m], o[:m].astype(np.float16))
+    assert np.all(np.abs(o16[:m].astype(np.float64) - ref) <= bound + np.abs(ref) * 2.0 ** -11 + 2.0 ** -24)

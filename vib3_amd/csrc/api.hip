@@ -37,7 +37,7 @@ int int4_flat(const void* x, int x_dt, const void* d0, const void* s0, const voi
     a.flat0 = MatRef{nullptr, (const uint8_t*)d0, (const uint16_t*)s0, 0, m, 0};
     a.flat1 = dual ? MatRef{nullptr, (const uint8_t*)d1, (const uint16_t*)s1, 0, m, 0} : a.flat0;
     a.out = out; a.out_dt = out_dt; a.out_stride = 0;
-    return launch_rows(a, dual, st);
+    return !dual && flat_down_ok(a) ? launch_flat_down(a, st) : launch_rows(a, dual, st);
   }
   GenericArgs a{x, x_dt, k, m, g, sdt, (const uint8_t*)d0, (const uint16_t*)s0,
                 (const uint8_t*)d1, (const uint16_t*)s1, out, out_dt};

@@ -831,7 +831,9 @@ __device__ __forceinline__ float lanes_sum(float v) {
 #endif
 constexpr int kDownScalarSlots = 16;  // most slots whose page addresses k_down_rows keeps in SGPRs
 
-template <int R, int J, int NB, bool ONE>  // ONE: the whole row in one pass (cpr <= CPP)
+// FLAT: one matrix at an address the host knows times one f16 vector (no tables, no weights; f16 or
+// f32 output).
+template <int R, int J, int NB, bool ONE, bool FLAT = false>  // ONE: the whole row in one pass (cpr <= CPP)
 __global__ __launch_bounds__(512) void k_down_rows(DownArgs a) {
   VIB3_TRACE_POINT(0);
   extern __shared__ uint4 lds[];
@@ -842,7 +844,7 @@ __global__ __launch_bounds__(512) void k_down_rows(DownArgs a) {
   const int grp = lane / L, sub = lane % L;
   const int cpr = a.K / 32, pk = a.K / 2, ng = (a.K + a.g - 1) / a.g;
   const int P = ONE ? 1 : (cpr + CPP - 1) / CPP;  // passes per slot
-  const int ns = a.nslots, top_k = a.top_k;
+  const int ns = FLAT ? 1 : a.nslots, top_k = FLAT ? 0 : a.top_k;
   const int CT = ONE ? CPP : cpr;  // chunks per slot in LDS (one pass: zero past cpr)
   uint4* xq = lds;                                       // [ns][4][CT] pair words
   float* xsum = (float*)(lds + (size_t)ns * 4 * CT);     // [ns][CT] offset term
@@ -857,22 +859,22 @@ __global__ __launch_bounds__(512) void k_down_rows(DownArgs a) {
   // pages hold whole row groups, the address of the page holding this wave's rows: the loop
   // then reads no page table (a scalar table read per batch would delay every batch's loads
   // by its latency)
-  const bool group_pages = a.rpp % R == 0;
+  const bool group_pages = FLAT || a.rpp % R == 0;
   // With the gate/up kernel's list of page addresses, whole row groups per page and few slots,
   // the page addresses come through scalar loads (one round trip, no ids), which leaves the
   // vector memory counter to the activations: those go out first, and waiting for the
   // addresses does not wait for them.
   const bool scalar_pages =
-      VIB3_DOWN_SCALAR_PAGES && a.bases && group_pages && ns <= kDownScalarSlots;
+      !FLAT && VIB3_DOWN_SCALAR_PAGES && a.bases && group_pages && ns <= kDownScalarSlots;
   const int r0 = min(R * g0, a.M - 1);
   const int page0 = (int)(((uint64_t)(uint32_t)r0 * a.magic) >> 32);  // page of this wave's rows
-  uint64_t my_t = 0, my_base = 0;
+  uint64_t my_t = 0, my_base = FLAT ? (uint64_t)(uintptr_t)a.flat : 0;
   float my_w = 1.0f;
-  if (lane < ns) {
+  if (!FLAT && lane < ns) {
     if (lane < top_k) my_w = a.wts[lane];
     else if (a.shared_w) my_w = a.shared_w[lane - top_k];  // sigmoid gate of a shared expert
   }
-  if (!scalar_pages && lane < ns) {
+  if (!FLAT && !scalar_pages && lane < ns) {
     const uint64_t* t =
         lane < top_k ? a.routed_table + ((size_t)a.ids[lane] * 3 + 2) * a.max_pages
                      : a.shared_table + ((size_t)(lane - top_k) * 3 + 2) * a.max_pages;
@@ -961,9 +963,9 @@ __global__ __launch_bounds__(512) void k_down_rows(DownArgs a) {
     }
     if (q.p == P - 1) {  // the slot's last pass: its row sums, rounded, into the combine
       float dsum = lanes_sum<L>(acc) * kTwo24;
-      if (a.round_f16) dsum = (float)(half_t)dsum;
+      if (!FLAT && a.round_f16) dsum = (float)(half_t)dsum;
       const float w = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_w), q.s));
-      const float next = add_mul_rn(o, w, dsum);  // weighted_accumulate_f32 in slot order
+      const float next = FLAT ? dsum : add_mul_rn(o, w, dsum);  // weighted_accumulate_f32 in slot order
       o = keep ? next : o;                         // (engine.rs:5262-5302)
       acc = 0.0f;
     }
@@ -1092,6 +1094,13 @@ __global__ __launch_bounds__(512) void k_down_rows(DownArgs a) {
   // stored after the loop: a store inside it would share the load counter with the weight
   // loads, and the compiler then waits for all of them at the loop head
   const int r = R * g0 + grp;
+  if (FLAT) {
+    if (sub == 0 && r < a.M) {
+      if (a.out_dt == VIB3_DT_F16) ((uint16_t*)a.out)[r] = f32_to_f16_bits(o);
+      else a.out[r] = o;
+    }
+    return;
+  }
   if (sub == 0 && r < a.M) a.out[r] = a.residual ? a.residual[r] + o : o;  // engine.rs:5302
   advance_router_tag(a.gen_word);
   VIB3_TRACE_POINT(3);
@@ -1458,7 +1467,7 @@ static size_t down_rows_lds(int nslots, int chunks) {
   return (size_t)nslots * chunks * (64 + 4);
 }
 
-template <int R, int J, bool ONE>
+template <int R, int J, bool ONE, bool FLAT = false>
 static void launch_down_rows_t(DownArgs& a, hipStream_t s, KTime t) {
   // One row group per wave, and as many waves per workgroup as make one workgroup per CU
   // (2..8): every CU streams the same share of the weights, and stages the activations once.
@@ -1468,7 +1477,7 @@ static void launch_down_rows_t(DownArgs& a, hipStream_t s, KTime t) {
   wpb = wpb < 2 ? 2 : wpb > 8 ? 8 : wpb;
   const int blocks = (groups + wpb - 1) / wpb;
   const int chunks = ONE ? kWave / R * J : a.K / 32;
-  hipExtLaunchKernelGGL((k_down_rows<R, J, kDownRowsBuffers, ONE>), dim3((unsigned)blocks),
+  hipExtLaunchKernelGGL((k_down_rows<R, J, kDownRowsBuffers, ONE, FLAT>), dim3((unsigned)blocks),
                         dim3(64 * wpb), (unsigned)down_rows_lds(a.nslots, chunks), s, t.start,
                         t.stop, 0, a);
 }
@@ -1480,6 +1489,31 @@ static void launch_down_rows_j(DownArgs& a, int cpr, hipStream_t s, KTime t) {
   else if (cpr <= 2 * L) launch_down_rows_t<R, 2, true>(a, s, t);
   else if (cpr <= 4 * L) launch_down_rows_t<R, 4, true>(a, s, t);
   else launch_down_rows_t<R, 4, false>(a, s, t);
+}
+
+// One flat matrix of 8192 < k, f16 activation: k_down_rows with one slot. k_int4_rows would need more
+// than four chunks per lane in registers, and k_int4_rows_ksplit, which splits k over two waves, reads
+// and converts the activation once per wave: 4096 x 14336 10.1 us there, 9.0 us here;
+// 512 x 8224 9.0 and 5.2; 7168 x 14336 14.4 either way. False where
+// the rows and scales are not one page, the staged activation exceeds 64 KB or rows exceed
+// page_magic's range.
+bool flat_down_ok(const RowsArgs& a) {
+  const int cpr = a.K / 32, pk = a.K / 2;
+  return a.x_dt == VIB3_DT_F16 && cpr > 4 * kWave && a.M < 65536 &&
+         down_rows_lds(1, cpr) <= 64 * 1024 &&
+         (const uint8_t*)a.flat0.scales == a.flat0.data + (size_t)a.M * pk;
+}
+
+int launch_flat_down(const RowsArgs& a, hipStream_t s) {
+  DownArgs d{};
+  d.h = a.x; d.h_dt = a.x_dt; d.K = a.K; d.M = a.M; d.g = a.g; d.sdt = a.sdt; d.nslots = 1;
+  d.rpp = a.M; d.magic = page_magic(a.M); d.flat = a.flat0.data;
+  d.out = (float*)a.out; d.out_dt = a.out_dt;
+  const int waves = 6 * device_cus();
+  if (a.M / 4 >= waves) launch_down_rows_t<4, 4, false, true>(d, s, KTime{});
+  else if (a.M / 2 >= waves) launch_down_rows_t<2, 4, false, true>(d, s, KTime{});
+  else launch_down_rows_t<1, 4, false, true>(d, s, KTime{});
+  VIB3_RETURN_LAUNCH();
 }
 
 int launch_down(DownArgs a, hipStream_t s, KTime t) {

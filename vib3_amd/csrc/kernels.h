@@ -134,6 +134,8 @@ struct DownArgs {
   const float* residual;  // out = residual + sum, or null
   const float* shared_w;  // [nslots - top_k] weights of the shared experts, or null (1.0)
   uint32_t* gen_word;     // router tag word advanced by block 0 (fused routing), or null
+  const uint8_t* flat;    // launch_flat_down: the matrix' page
+  int out_dt;             // launch_flat_down: type of out
 };
 
 // The down kernel, the layer's last, advances the router tag for the next launch. It runs
@@ -161,6 +163,9 @@ bool rows_write_bases(const RowsArgs& a);
 bool rows_fuse_prologue(const RowsArgs& a);
 int launch_down(DownArgs a, hipStream_t s, KTime t = {});
 int launch_generic(GenericArgs a, bool dual, hipStream_t s);
+// one flat matrix (a.flat0) with a long k through the down kernel, where flat_down_ok says so
+bool flat_down_ok(const RowsArgs& a);
+int launch_flat_down(const RowsArgs& a, hipStream_t s);
 // RMSNorm of x into xn (norm_w set) and the shared experts' sigmoid gates (gate_w set).
 int launch_moe_prologue(const void* x, int x_dt, const uint16_t* norm_w, float eps, int D,
                         float* xn, const uint16_t* gate_w, int ns, float* shared_w,
