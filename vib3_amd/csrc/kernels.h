@@ -134,8 +134,6 @@ struct DownArgs {
   const float* residual;  // out = residual + sum, or null
   const float* shared_w;  // [nslots - top_k] weights of the shared experts, or null (1.0)
   uint32_t* gen_word;     // router tag word advanced by block 0 (fused routing), or null
-  const uint8_t* flat;    // launch_flat_down: the matrix' page
-  int out_dt;             // launch_flat_down: type of out
 };
 
 // The down kernel, the layer's last, advances the router tag for the next launch. It runs
@@ -163,6 +161,8 @@ bool rows_write_bases(const RowsArgs& a);
 bool rows_fuse_prologue(const RowsArgs& a);
 int launch_down(DownArgs a, hipStream_t s, KTime t = {});
 int launch_generic(GenericArgs a, bool dual, hipStream_t s);
+// one page with unaligned rows (k >= 32, g a multiple of 32)
+int launch_ragged(const GenericArgs& a, bool dual, hipStream_t s);
 // one flat matrix (a.flat0) with a long k through the down kernel, where flat_down_ok says so
 bool flat_down_ok(const RowsArgs& a);
 int launch_flat_down(const RowsArgs& a, hipStream_t s);
