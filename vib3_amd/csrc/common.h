@@ -318,18 +318,18 @@ __device__ __forceinline__ void mat_row(const MatRef& m, int r, int pk, int ng, 
 #define VIB3_WAIT_VM(n) __builtin_amdgcn_s_waitcnt(0x0F70 | ((n) & 15) | (((n) >> 4) << 14))
 
 // Timeline probes for kernel-internal phases: compiled in only when VIB3_TRACE is defined (a
-// profiling build; the buffer pointer is set per translation unit by vib3_trace_set in
-// int4_gemv.hip); each probe stores the 100 MHz real-time counter for (workgroup, point).
+// profiling build; the buffer pointer is set per translation unit, by vib3_trace_set in
+// int4_gemv.hip and vib3_trace_set_fp4 in fp4_fused.hip); each probe stores the 100 MHz real-time
+// counter for (workgroup, point). Translation units that share a probed kernel's source or a probed
+// header without a setter of their own (int4_pages.hip, router.hip) keep a null pointer: there a
+// probe stores nothing.
 #ifdef VIB3_TRACE
 static __device__ uint64_t* vib3_trace_buf;
-#define VIB3_TRACE_POINT(k)                                                          \
-  do {                                                                               \
-    if (threadIdx.x == 0) vib3_trace_buf[blockIdx.x * 16 + (k)] = __builtin_amdgcn_s_memrealtime(); \
-  } while (0)
-#define VIB3_TRACE_VALUE(k, v)                                                       \
-  do {                                                                               \
-    if (threadIdx.x == 0) vib3_trace_buf[blockIdx.x * 16 + (k)] = (uint64_t)(v);       \
-  } while (0)
+__device__ __forceinline__ void trace_store(unsigned block, int k, uint64_t v) {
+  if (threadIdx.x == 0 && vib3_trace_buf) vib3_trace_buf[block * 16 + k] = v;
+}
+#define VIB3_TRACE_POINT(k) trace_store(blockIdx.x, (k), __builtin_amdgcn_s_memrealtime())
+#define VIB3_TRACE_VALUE(k, v) trace_store(blockIdx.x, (k), (uint64_t)(v))
 #else
 #define VIB3_TRACE_VALUE(k, v) \
   do {                         \

@@ -549,12 +549,8 @@ __global__ __launch_bounds__(256) void k_fp4_rms_quant(const float* x, const uin
 // and k quarter w & 3 of both matrices; the quarters meet in LDS, and the 32 rows, one E8M0
 // group of h, are quantized and written split-half.
 #ifdef VIB3_TRACE  // (2-D grid: one probe row per workgroup, y-major)
-#define FP4_TRACE(k)                                                                     \
-  do {                                                                                   \
-    if (threadIdx.x == 0)                                                                \
-      vib3_trace_buf[(blockIdx.y * gridDim.x + blockIdx.x) * 16 + (k)] =                 \
-          __builtin_amdgcn_s_memrealtime();                                              \
-  } while (0)
+#define FP4_TRACE(k) \
+  trace_store(blockIdx.y * gridDim.x + blockIdx.x, (k), __builtin_amdgcn_s_memrealtime())
 #else
 #define FP4_TRACE(k) \
   do {               \
