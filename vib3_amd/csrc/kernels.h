@@ -6,6 +6,7 @@
 #include <stdint.h>
 
 #include "common.h"
+#include "device_cache.h"
 #include "../../include/vib3_hip.h"
 
 namespace vib3 {
@@ -176,16 +177,15 @@ constexpr int kMaxExperts = 4096;
 // Resident workgroups per CU for a kernel at a block size, and the CU count (cached per device;
 // plain host queries, no allocation).
 static inline int device_cus() {
-  static int cus[64] = {0};
+  static DeviceCache cus;
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cus[dev]) {
+  return cus.get(dev, [dev] {
     int n = 0;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
       n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
+    return n;
+  });
 }
 
 template <typename K>

@@ -1067,14 +1067,14 @@ __global__ __launch_bounds__(256) void k_mx_combine(const uint16_t* d, const flo
 }
 
 // One row-path kernel at its resident grid, cached per instantiation and device (each
-// <GATEUP, NCH, NT> variant has its own register budget and therefore its own occupancy).
+// <GATEUP, NCH, NT> variant has its own register budget and therefore its own occupancy). Called
+// with and without the side streams' lock.
 template <bool GATEUP, int NCH, int NT>
 static void mx_launch_rows_one(const MxArgs& a, hipStream_t st) {
-  static int grid[64] = {0};
+  static DeviceCache grid;
   int dev = 0;
   (void)hipGetDevice(&dev);
-  int& g = grid[dev & 63];
-  if (!g) g = resident_blocks(k_mx_rows<GATEUP, NCH, NT>, 256);
+  const int g = grid.get(dev, [] { return resident_blocks(k_mx_rows<GATEUP, NCH, NT>, 256); });
   hipLaunchKernelGGL((k_mx_rows<GATEUP, NCH, NT>), dim3((unsigned)g), dim3(256), 0, st, a);
 }
 
@@ -1099,8 +1099,9 @@ static void mx_launch_rows(const MxArgs& a, int K, bool merged, hipStream_t st1,
 // The paths are independent until the combine. Larger batches run them on streams of the library
 // beside the caller's (three per device, default priority), forked after the grouping and joined
 // before the combine with events, so each path fills the others' ramps and tails (mx_streams says
-// when). Enqueueing is serialised by a lock (the side streams and their events are shared by every
-// call on that device); under graph capture the fork and join become graph edges.
+// when). Enqueueing of such batches is serialised by a lock (the side streams and their events are
+// shared by every call on that device); batches on the caller's stream alone share no host state but
+// the launch-size caches. Under graph capture the fork and join become graph edges.
 struct MxSide {
   hipStream_t st = nullptr, st2 = nullptr;  // one-token and two-token row paths
   hipStream_t st3 = nullptr;                // wide items
