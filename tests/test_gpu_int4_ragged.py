@@ -57,3 +57,57 @@ def test_ragged_pages(k, m, g, sdt, adt, pshift, xshift):
     assert np.linalg.norm(t[:m] - ref2) <= 5e-5 * np.linalg.norm(ref2)
     assert np.array_equal(out16.cpu().numpy()[:m], o[:m].astype(np.float16))
     assert (o[m:] == 7.5).all() and (t[m:] == 7.5).all()
+
+
+def _page(codes, scales):
+    """One INT4 page from codes [m][k] (0..15) and scales [m][groups] as bf16 bits."""
+    m, k = codes.shape
+    c = np.zeros((m, 2 * ((k + 1) // 2)), dtype=np.uint8)
+    c[:, :k] = codes
+    return np.concatenate([(c[:, ::2] | (c[:, 1::2] << 4)).ravel(), scales.astype(np.uint16).view(np.uint8).ravel()])
+
+
+@pytest.mark.parametrize("k,m", [(1000, 8), (2049, 8), (8193, 8), (1000, 8 * 1024 + 5)])
+def test_ragged_large_and_infinite_values(k, m):
+    """Terms x ((q - 8) scale) far below the f32 limit whose x (q - 8) is above it sum to what the terms
+    do; an infinite activation comes through as in the term-by-term sum; scales that are no positive
+    number read as 1/8, also the last group's, which lanes without a chunk of their own load too."""
+    from vib3_amd import _lib
+    print(f"case: ragged large values k={k} m={m}", flush=True)
+    g = 32
+    rng = np.random.default_rng(k)
+    ng = -(-k // g)
+    codes = rng.integers(0, 16, (m, k))
+    scales = np.full((m, ng), 0x3080)  # bf16 2^-30
+    scales[0, ng - 1], scales[1, 5], scales[2, ng - 2] = 0x7F80, 0x7FC0, 0xFF80  # inf, NaN, -inf
+    x = rng.standard_normal(k).astype(np.float32)
+    big, bad = x.copy(), x.copy()
+    big[40:72] = 2.0e38            # x (q - 8) passes 2^128, every term stays below 2^125
+    codes[4, 40:72] = 15
+    bad[k - 1] = np.inf
+    codes[:, k - 1] = np.where(np.arange(m) == 3, 8, 9)  # row 3: inf * 0
+    s = (scales.astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+    s = np.where(np.isfinite(s) & (s > 0), s, 0.125)
+    page = torch.from_numpy(_page(codes, scales)).cuda()
+    for xv in (x, big, bad):
+        with np.errstate(invalid="ignore"):
+            terms = xv.astype(np.float64) * ((codes - 8) * s.repeat(g, 1)[:, :k])
+            ref = terms.sum(1)
+            # k f32 additions in any order and one product per term: (k + 2) roundings
+            bound = (k + 2) * 2.0 ** -24 * np.abs(terms).sum(1)
+        xd = torch.from_numpy(xv).cuda()
+        out = torch.empty(m, dtype=torch.float32, device="cuda")
+        two = torch.empty(m, dtype=torch.float32, device="cuda")
+        st = torch.cuda.current_stream().cuda_stream
+        _lib.call("vib3_launch_partial_matmul_int4_ex", xd.data_ptr(), O.F32, page.data_ptr(), out.data_ptr(),
+                  _lib.DT_F32, k, m, g, O.BF16, st)
+        _lib.call("vib3_launch_partial_swiglu_int4_ex", xd.data_ptr(), O.F32, page.data_ptr(), page.data_ptr(),
+                  two.data_ptr(), _lib.DT_F32, k, m, g, O.BF16, st)
+        torch.cuda.synchronize()
+        o, t = out.cpu().numpy(), two.cpu().numpy()
+        fin = np.isfinite(ref)
+        assert np.array_equal(np.isnan(o), np.isnan(ref)) and np.array_equal(np.isinf(o), np.isinf(ref)), (o, ref)
+        assert (np.abs(o[fin] - ref[fin]) <= bound[fin]).all(), (o, ref)
+        with np.errstate(invalid="ignore", over="ignore"):
+            sw = (o / (np.float32(1) + np.exp(-o))) * o  # silu(gate) * up of the same sums
+        assert np.array_equal(np.isfinite(t), np.isfinite(sw)), (t, sw)

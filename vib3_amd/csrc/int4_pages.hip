@@ -126,12 +126,19 @@ __global__ __launch_bounds__(128) void k_int4_ragged(GenericArgs a) {
       }
     }
   };
+  auto store = [&](int row, const float (&t)[NS]) {
+    const float v = DUAL ? (t[NS - 1] / (1.0f + expf(-t[NS - 1]))) * t[0] : t[0];
+    if (a.out_dt == VIB3_DT_F16) ((uint16_t*)a.out)[row] = f32_to_f16_bits(v);
+    else ((float*)a.out)[row] = v;
+  };
+  uint64_t again = 0;
   int rg = (int)blockIdx.x * 2 + wave;
   if (ONE) {
     issue(min(rg * R + rr, M - 1), 0);
     load_x(0);
   }
-  for (bool first = true; rg < groups; rg += stride, first = false) {
+  for (int turn = 0; rg < groups; rg += stride, turn++) {
+    const bool first = turn == 0;
     const int row = rg * R + rr;
     float acc[NS];
 #pragma unroll
@@ -149,19 +156,32 @@ __global__ __launch_bounds__(128) void k_int4_ragged(GenericArgs a) {
     }
 #pragma unroll
     for (int m = 0; m < NS; m++) {
-      float v = acc[m];
-      v += dpp<0xB1>(v);
-      v += dpp<0x4E>(v);
-      v += dpp<0x141>(v);
-      v += dpp<0x140>(v);
-      if (L >= 32) v += __shfl_xor(v, 16);
-      if (L >= 64) v += __shfl_xor(v, 32);
-      acc[m] = v;
+      acc[m] = lanes_sum<L>(acc[m]);
+      // (infinite or no number, which a sum stays once it is; a row's lanes agree)
+      if (!(__builtin_fabsf(acc[m]) <= __FLT_MAX__)) again |= 1ull << (turn & 63);
     }
-    if (sub == 0 && row < M) {
-      const float v = DUAL ? (acc[NS - 1] / (1.0f + expf(-acc[NS - 1]))) * acc[0] : acc[0];
-      if (a.out_dt == VIB3_DT_F16) ((uint16_t*)a.out)[row] = f32_to_f16_bits(v);
-      else ((float*)a.out)[row] = v;
+    if (sub == 0 && row < M) store(row, acc);
+  }
+  // Rows whose sums overflowed, or whose terms are no finite numbers, term by term: with |x| above
+  // 2^120 a chunk's sum of x (q - 8) can overflow ahead of its scale where no x ((q - 8) scale) does.
+  // (After the loop: a branch inside it cost 0.3 us per launch. A bit stands for every 64th turn.)
+  if (__builtin_expect(again != 0, 0)) {
+    rg = (int)blockIdx.x * 2 + wave;
+    for (int turn = 0; rg < groups; rg += stride, turn++) {
+      const int row = rg * R + rr;
+      if (row >= M || !(again >> (turn & 63) & 1)) continue;
+      float t[NS];
+      for (int m = 0; m < NS; m++) {
+        float v = 0.0f;
+        for (int col = sub; col < K; col += L) {
+          const uint8_t b = d[m][(size_t)row * pk + (col >> 1)];
+          const int code = (col & 1) ? b >> 4 : b & 15;
+          const uint16_t sc = *(__attribute__((address_space(1))) const u16_u*)(s[m] + 2 * ((size_t)row * ng + col / a.g));
+          v = __builtin_fmaf(load_act(a.x, a.x_dt, col), (float)(code - 8) * decode_scale(sc, a.sdt), v);
+        }
+        t[m] = lanes_sum<L>(v);
+      }
+      if (sub == 0) store(row, t);
     }
   }
 }
