@@ -190,7 +190,7 @@ typedef struct vib3_moe_int4_layer {
     int x_dtype;
     int hidden; /* k of gate/up, rows of down */
     int inter;  /* rows of gate/up, k of down */
-    int group_size;
+    int group_size; /* columns per scale: a multiple of 32, or one group per row */
     int scale_dtype;
     /* router; when router_w is NULL the experts come from in_ids / in_weights (device) */
     const void *router_w; /* [num_experts][hidden] */

@@ -20,15 +20,18 @@ inline bool valid_scale_dt(int dt) { return dt == VIB3_DT_F16 || dt == VIB3_DT_B
 inline bool valid_out_dt(int dt) { return dt == VIB3_DT_F32 || dt == VIB3_DT_F16; }
 inline size_t round_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
-// One flat INT4 matrix (or up/gate pair) times a vector: the fast kernel when the shape and
-// alignment allow 16-byte chunk loads, otherwise the generic kernel.
+// The chunk kernels read one scale per 32 columns: each chunk of 32 must lie in one group.
+inline bool chunk_groups(int g, int k) { return g % 32 == 0 || g >= k; }
+
+// One flat INT4 matrix (or up/gate pair) times a vector: the fast kernel when the shape, the groups
+// and the alignment allow 16-byte chunk loads, otherwise the unaligned or the generic kernel.
 int int4_flat(const void* x, int x_dt, const void* d0, const void* s0, const void* d1,
               const void* s1, void* out, int out_dt, int k, int m, int g, int sdt, bool dual,
               hipStream_t st) {
   if (k <= 0 || m < 0 || g <= 0) return VIB3_ERR_BAD_COUNT;
   if (!x || !d0 || !s0 || !out || (dual && (!d1 || !s1))) return VIB3_ERR_BAD_POINTER;
   if (m == 0) return 0;
-  const bool fast = (k % 32 == 0) && (k / 32 <= 16 * kWave) && aligned16(d0) &&
+  const bool fast = (k % 32 == 0) && chunk_groups(g, k) && (k / 32 <= 16 * kWave) && aligned16(d0) &&
                     (!dual || aligned16(d1)) && aligned16(x) && ((uintptr_t)s0 % 2 == 0) &&
                     (!dual || (uintptr_t)s1 % 2 == 0);
   if (fast) {
@@ -385,6 +388,8 @@ static int moe_int4_layer(const vib3_moe_int4_layer* L, void* stream, int only,
   const int nslots = L->top_k + L->num_shared;
   if (nslots <= 0 || nslots > 16 || L->top_k > 64) return VIB3_ERR_BAD_COUNT;
   if (L->hidden % 32 || L->inter % 32) return VIB3_ERR_UNSUPPORTED;
+  if (!chunk_groups(L->group_size, L->hidden) || !chunk_groups(L->group_size, L->inter))
+    return VIB3_ERR_UNSUPPORTED;
   if (L->hidden >= 65536 || L->inter >= 65536) return VIB3_ERR_UNSUPPORTED;  // page_magic range
   for (int s = 0; s < 3; s++)
     if (L->rows_per_page[s] <= 0) return VIB3_ERR_BAD_COUNT;

@@ -783,7 +783,7 @@ __global__ __launch_bounds__(WIDE ? 1024 : 640) void k_down_combine(DownArgs a) 
 }
 
 // ------------------------------------------------------------------------- k_int4_generic
-// (k < 32 or a group size that is no multiple of 32)
+// (k < 32 or a group size that is no multiple of 32; aligned pages too, see int4_flat)
 
 template <bool DUAL>
 __global__ __launch_bounds__(256) void k_int4_generic(GenericArgs a) {
