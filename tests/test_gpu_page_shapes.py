@@ -98,3 +98,16 @@ def test_scalar(k, m):
     assert np.all(np.abs(g32[:m] - want) <= k * 2.0 ** -24 * mags + 1e-30)
     assert np.all(np.abs(g16[:m].astype(np.float64) - want) <= np.abs(want) * 2.0 ** -11 + 2.0 ** -24 + k * 2.0 ** -23 * mags)
     assert (g32[m:] == 7.5).all() and (g16[m:] == 7.5).all()
+
+
+# Both sides of the lines between the row kernel and the staged one (16-row workgroups): short rows, many
+# rows of each lane count, pairs and tiled pages earlier than single row-major ones; rows that are no
+# whole workgroup, a staged activation near the longest the f32-input form takes.
+CHOICE = [(64, 64), (1024, 65), (1056, 64), (1056, 65), (1024, 16), (2048, 2560), (2048, 2576), (2560, 6144), (2560, 6161),
+          (4096, 6160), (3072, 12288), (3072, 12304), (4160, 6144), (4160, 6160), (4160, 8208), (4128, 12289),
+          (20032, 6160)]
+
+
+@pytest.mark.parametrize("k,m", CHOICE)
+def test_block_scaled_kernel_choice(k, m):
+    test_block_scaled(k, m)

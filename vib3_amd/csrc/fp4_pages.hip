@@ -267,6 +267,57 @@ __global__ __launch_bounds__(256) void k_fp4_page_rows(PageGemvArgs a) {
   }
 }
 
+// One group's 16 split-half bytes as the LDS pair layout group_dot reads.
+__device__ __forceinline__ void put_group(uint4* pairs, int* ex, int g, uint4 w, int e) {
+  f16x2 p[16];
+  decode_group(w, p);
+#pragma unroll
+  for (int q = 0; q < 4; q++)
+    pairs[(size_t)g * 4 + q] =
+        make_uint4(__builtin_bit_cast(uint32_t, p[4 * q]), __builtin_bit_cast(uint32_t, p[4 * q + 1]),
+                   __builtin_bit_cast(uint32_t, p[4 * q + 2]), __builtin_bit_cast(uint32_t, p[4 * q + 3]));
+  ex[g] = e;
+}
+
+// The same GEMV with the activation staged: workgroup = 16 rows, 16 lanes per row (a lane takes
+// groups l, l + 16, ...), the activation decoded once per workgroup into LDS pairs and exponents. One
+// workgroup per 16 rows keeps every wave short and lets the hardware balance them, which wins where
+// k_fp4_page_rows has too few groups per lane (short rows) or too many rows per wave (see page_staged).
+template <int LAY, bool FULL, int NS>
+__global__ __launch_bounds__(256) void k_fp4_page_staged(PageGemvArgs a) {
+  extern __shared__ uint4 lds[];
+  const int G = a.K / 32, tid = (int)threadIdx.x;
+  // the arguments' two cache lines in one round trip (K lies in the second: fetching `act` behind it
+  // cost 0.25 us of 2.5 to 4)
+  asm volatile("" ::"s"(a.K), "s"(a.act));
+  uint4* pairs = lds;                      // [G][4]
+  int* ex = (int*)(lds + (size_t)G * 4);   // [G]
+  for (int g = tid; g < G; g += 256)
+    put_group(pairs, ex, g, *(const uint4*)(a.act + (size_t)g * 16), a.act_sc[g]);
+  __syncthreads();
+  const int gl = tid & 15, row = (int)blockIdx.x * 16 + (tid >> 4);
+  const int rc = row < a.M ? row : a.M - 1;
+  double acc[NS];
+#pragma unroll
+  for (int m = 0; m < NS; m++) acc[m] = 0.0;
+  for (int g = gl; g < G; g += 16) {
+    const double ea = pow2d(ex[g] - 127);
+#pragma unroll
+    for (int m = 0; m < NS; m++) {
+      const uint4 w = *(const uint4*)group_ptr<LAY>(a.w[m], rc, g, a.K);
+      const uint16_t sw = a.s[m][(size_t)rc * G + g];
+      const double ws = FULL ? (double)bf16_to_f32(sw) : pow2d((int)((sw >> 7) & 0xff) - 127);
+      acc[m] = fma((double)group_dot(w, pairs + (size_t)g * 4), ws * ea, acc[m]);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < NS; m++)
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) acc[m] += shfl_xor_d(acc[m], o);
+  if (gl == 0 && row < a.M)
+    a.out[row] = NS == 1 ? (float)acc[0] : swiglu_fp4((float)acc[NS - 1], (float)acc[0]);
+}
+
 struct ScalarArgs {
   const void* x;          // f32 or f16 [K]
   const uint8_t* w[2];    // sequential codes [M][K/2]
@@ -377,6 +428,25 @@ PageShape page_shape(int M, int G) {
   return p;
 }
 
+// Whether a page with quantized activations takes k_fp4_page_staged. us per launch, weights from HBM,
+// staged / row kernel:
+//   * short rows, where a launch's fixed chain decides: K = 1024 520 rows 3.2 / 3.4, pairs 3.8 / 3.9
+//     (16 rows 3.2 / 2.6), K = 512 2.5 / 3.1;
+//   * many rows, where the row kernel's waves walk several row groups: K = 2048 2064 rows 4.6 / 4.3,
+//     8192 5.4 / 5.7, pairs 5.5 / 5.3 and 5.7 / 6.0 (3072 rows); K = 2560 7168 rows 5.9 / 5.9, 16384
+//     7.8 / 9.3; K = 4096 12288 rows 10.2 / 9.2, 16384 10.8 / 11.4, pairs of 6144 9.9 / 9.0, 8192 10.6 / 10.8;
+//     K = 7168 12288 rows 16.3 / 14.6, pairs of 8192 16.4 / 16.4, 10240 18.6 / 19.7;
+//   * tiled pages, whose 64 lanes per row (K > 4096) take 32 bytes of each 128-byte line, earlier:
+//     K = 7168 6144 rows 12.2 / 12.0, 7168 12.8 / 13.2, 12288 16.4 / 21.6.
+bool page_staged(int lay, int ns, int K, int M) {
+  if (K <= 1024) return ns == 1 || M > 64;
+  if (K <= 2048) return M > 2560;
+  if (K <= 2560) return M > 6144;
+  if (K <= 4096) return M > (ns == 2 ? 6144 : 12288);
+  if (K >= 8192 && lay != kLayTiled) return ns == 1 && M > 14336;
+  return M > (lay == kLayTiled ? 6144 : ns == 2 ? 8192 : 12288);
+}
+
 int page_gemv(int lay, bool full, int ns, const void* act, const void* act_sc, const float* x,
               const void* w0, const void* s0, const void* w1, const void* s1, void* out, int K,
               int M, void* stream) {
@@ -388,16 +458,28 @@ int page_gemv(int lay, bool full, int ns, const void* act, const void* act_sc, c
     return VIB3_ERR_BAD_POINTER;
   if (M == 0) return 0;
   const int G = K / 32;
-  // K's limit (30816, or 23808 with f32 input): the whole decoded activation in 64 KB
+  // K's limit (30816, or 23808 with f32 input): the whole decoded activation in 64 KB (what
+  // k_fp4_page_staged holds)
   if ((size_t)G * 68 + (act ? 0 : (size_t)G * 20 + 32) > 65536) return VIB3_ERR_UNSUPPORTED;
   PageGemvArgs a{};
   a.act = (const uint8_t*)act; a.act_sc = (const uint8_t*)act_sc; a.x = x;
   a.w[0] = (const uint8_t*)w0; a.s[0] = (const uint16_t*)s0;
   a.w[1] = (const uint8_t*)w1; a.s[1] = (const uint16_t*)s1;
   a.out = (float*)out; a.K = K; a.M = M;
+  hipStream_t st = (hipStream_t)stream;
+  if (act && page_staged(lay, ns, K, M)) {
+#define VIB3_PAGE_STAGED(LY, F, N)                                                              \
+  hipLaunchKernelGGL((k_fp4_page_staged<LY, F, N>), dim3((unsigned)((M + 15) / 16)), dim3(256), \
+                     (unsigned)G * 68u, st, a)
+    if (lay == kLayTiled) VIB3_PAGE_STAGED(kLayTiled, false, 1);
+    else if (full) VIB3_PAGE_STAGED(kLayRowSplit, true, 1);
+    else if (ns == 2) VIB3_PAGE_STAGED(kLayRowSplit, false, 2);
+    else VIB3_PAGE_STAGED(kLayRowSplit, false, 1);
+#undef VIB3_PAGE_STAGED
+    VIB3_RETURN_LAUNCH();
+  }
   const PageShape p = page_shape(M, G);
   const unsigned lds = act ? 0u : (unsigned)G * 20u;
-  hipStream_t st = (hipStream_t)stream;
 #define VIB3_PAGE_L(LY, F, N, LL, O) \
   hipLaunchKernelGGL((k_fp4_page_rows<LY, F, N, LL, O>), dim3(p.grid), dim3(p.block), lds, st, a)
 #define VIB3_PAGE_GEMV(LY, F, N)                        \
