@@ -1,4 +1,4 @@
-"""The unaligned INT4 page kernel at its edges: k from one chunk up, odd k, k one past a multiple of
+"""The unaligned INT4 page kernels at their edges: k from one chunk up, odd k, k one past a multiple of
 32, the k at which a row takes 16 / 32 / 64 lanes and several passes, few and many rows, pages and
 activations at odd addresses with NaNs around the activation (no column outside it may count)."""
 import numpy as np
@@ -57,6 +57,18 @@ def test_ragged_pages(k, m, g, sdt, adt, pshift, xshift):
     assert np.linalg.norm(t[:m] - ref2) <= 5e-5 * np.linalg.norm(ref2)
     assert np.array_equal(out16.cpu().numpy()[:m], o[:m].astype(np.float16))
     assert (o[m:] == 7.5).all() and (t[m:] == 7.5).all()
+
+
+# Both sides of the lines between this kernel and the per-column one: rows of two and three chunks, pairs
+# of four and five, and pairs of many rows.
+CHOICE = [(64, 300, 32, O.BF16, O.F16, 8, 1), (65, 300, 32, O.BF16, O.F32, 0, 0), (96, 9, 64, O.F16, O.BF16, 1, 0),
+          (128, 130, 32, O.BF16, O.F16, 2, 0), (129, 130, 32, O.BF16, O.F16, 0, 1), (100, 8191, 32, O.BF16, O.F32, 0, 0),
+          (100, 8192, 32, O.BF16, O.F32, 0, 0), (127, 8193, 64, O.F16, O.F16, 0, 0)]
+
+
+@pytest.mark.parametrize("k,m,g,sdt,adt,pshift,xshift", CHOICE)
+def test_ragged_kernel_choice(k, m, g, sdt, adt, pshift, xshift):
+    test_ragged_pages(k, m, g, sdt, adt, pshift, xshift)
 
 
 def _page(codes, scales):

@@ -12,7 +12,7 @@
 //                    single GEMV), used by the layer and by the partial_* launchers.
 // k_down_combine   — down projection of all expert slots for a block of output rows, with the
 //                    weighted sum over experts (fixed order, no atomics) in the epilogue.
-// k_int4_generic   — any k and g; one wave per row.
+// k_int4_generic   — any k and g, one wave per row: short unaligned rows, odd group sizes.
 // k_down_rows      — the same down projection from activations staged in LDS (down_rows.h).
 #include <stdlib.h>
 
@@ -783,7 +783,7 @@ __global__ __launch_bounds__(WIDE ? 1024 : 640) void k_down_combine(DownArgs a) 
 }
 
 // ------------------------------------------------------------------------- k_int4_generic
-// (k < 32 or a group size that is no multiple of 32; aligned pages too, see int4_flat)
+// (rows of a few chunks, and group sizes that are no multiple of 32 whatever the alignment)
 
 template <bool DUAL>
 __global__ __launch_bounds__(256) void k_int4_generic(GenericArgs a) {
@@ -1014,9 +1014,14 @@ int launch_down(DownArgs a, hipStream_t s, KTime t) {
 
 int launch_generic(GenericArgs a, bool dual, hipStream_t s) {
   if (a.M <= 0) return 0;
-  if (a.K >= 32 && a.g % 32 == 0) {  // (rows of at least one whole chunk)
-    return launch_ragged(a, dual, s);
-  }
+  // k_int4_ragged needs rows of at least one whole chunk and one scale per chunk. Rows of a few chunks
+  // leave most of its 16 lanes per row idle behind a longer start: us per launch, this kernel / that
+  // one, k = 63: 520 rows 1.9 / 2.4, pairs 2.1 / 3.1, 14336 rows 4.3 / 4.8 and 5.6 / 6.1; k = 100: 520 rows
+  // 2.4 / 2.4, pairs 2.8 / 3.2, 4096 rows 3.5 / 4.0, 14336 rows 6.8 / 5.8; k = 129: pairs 3.2 / 3.3, 14336 rows
+  // 8.1 / 6.3 (f16 activations, pages from HBM).
+  const int chunks = (a.K + 31) / 32;
+  const bool short_rows = chunks <= 2 || (dual && chunks <= 4 && a.M < 8192);
+  if (!short_rows && a.g % 32 == 0) return launch_ragged(a, dual, s);
   dim3 grid((unsigned)((a.M + 3) / 4));
   if (dual) hipLaunchKernelGGL((k_int4_generic<true>), grid, dim3(256), 0, s, a);
   else hipLaunchKernelGGL((k_int4_generic<false>), grid, dim3(256), 0, s, a);

@@ -162,7 +162,7 @@ bool rows_write_bases(const RowsArgs& a);
 bool rows_fuse_prologue(const RowsArgs& a);
 int launch_down(DownArgs a, hipStream_t s, KTime t = {});
 int launch_generic(GenericArgs a, bool dual, hipStream_t s);
-// one page with unaligned rows (k >= 32, g a multiple of 32)
+// one page with unaligned rows (k > 64, g a multiple of 32)
 int launch_ragged(const GenericArgs& a, bool dual, hipStream_t s);
 // one flat matrix (a.flat0) with a long k through the down kernel, where flat_down_ok says so
 bool flat_down_ok(const RowsArgs& a);
