@@ -55,6 +55,13 @@ def test_weight_quantizer(m, k, shift):
     assert (d[shift + m * k // 2:] == 0xA5).all() and (s[m * k // 32:] == 0x5A5A).all()
 
 
+@pytest.mark.parametrize("m,k,shift", [(63, 4160, 0), (64, 4096, 0), (257, 1056, 0), (2, 131104, 0), (64, 4096, 1)])
+def test_weight_quantizer_kernel_choice(m, k, shift):
+    """Matrices just below and above the size from which a lane takes eight weights, with whole and
+    partial last blocks."""
+    test_weight_quantizer(m, k, shift)
+
+
 @pytest.mark.parametrize("m,k", [(16, 64), (48, 192), (16, 2048), (32, 2112), (16, 16384), (16, 16448)])
 def test_repack_row_to_tiled(m, k):
     from vib3_amd import kernels as K

@@ -464,7 +464,7 @@ __global__ __launch_bounds__(256) void k_fp4_weight_quant(const uint16_t* w, uin
   }
 }
 
-// The same, one lane per weight: input not 16-byte aligned or codes not 4-byte aligned.
+// The same, one lane per weight: small matrices, input not 16-byte aligned or codes not 4-byte aligned.
 __global__ __launch_bounds__(256) void k_fp4_weight_quant_any(const uint16_t* w, uint8_t* codes,
                                                               uint16_t* scales, long long n) {
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -955,7 +955,10 @@ int vib3_launch_fp16_to_nvfp4_weight(const void* input, void* out_data, void* ou
   if (!input || !out_data || !out_scales) return VIB3_ERR_BAD_POINTER;
   const long long n = (long long)M * K;
   if (n == 0) return 0;
-  if ((((uintptr_t)input & 15) | ((uintptr_t)out_data & 3)) == 0) {
+  // Eight weights per lane need 16-byte input and 4-byte code alignment, and enough weights to fill
+  // the card with workgroups of 8192 of them: us from HBM, one / eight weights per lane, 8192 weights
+  // 1.9 / 2.6, 65536 2.6 / 2.8, 262144 2.8 / 2.8, 524288 3.4 / 2.9.
+  if ((((uintptr_t)input & 15) | ((uintptr_t)out_data & 3)) == 0 && n >= 262144) {
     const long long n8 = n / 8, per = 256 * kWqUnroll;
     hipLaunchKernelGGL(k_fp4_weight_quant, dim3((unsigned)((n8 + per - 1) / per)), dim3(256), 0,
                        (hipStream_t)stream, (const uint16_t*)input, (uint8_t*)out_data,
