@@ -1,6 +1,7 @@
 """One INT4 page with k > 8192 and f16 activations: the staged-activation kernel (one chunk past four
 per lane, no multiple of a pass, the longest k its LDS holds, one to four rows per wave, few rows), and
-the shapes just outside it (scales not behind the rows, k past its LDS) that keep the split kernel."""
+the shapes just outside it (scales not behind the rows, k past its LDS, row counts at which the split
+kernel is faster) that keep the split kernel."""
 import numpy as np
 import pytest
 
@@ -11,6 +12,11 @@ torch = pytest.importorskip("torch")
 
 
 @pytest.mark.parametrize("k,m,g,sdt,apart", [
+    # both sides of the lines between the two kernels, and of those between 1, 2 and 4 rows per wave
+    (8224, 2049, 32, O.BF16, False), (8224, 4097, 32, O.F16, False), (8224, 8193, 32, O.BF16, False),
+    (12288, 14337, 128, O.F16, False), (14336, 7169, 128, O.F16, False), (18432, 4, 32, O.BF16, False),
+    (18432, 5, 32, O.BF16, False), (20480, 4100, 128, O.BF16, False), (24576, 4097, 128, O.F16, False),
+    (24576, 6145, 128, O.F16, False), (28672, 2049, 128, O.BF16, False),
     (8224, 1, 32, O.BF16, False), (8224, 523, 64, O.F16, False), (9216, 3073, 32, O.BF16, False),
     (14336, 6149, 128, O.F16, False), (30816, 5, 32, O.BF16, False), (30848, 5, 32, O.BF16, False),
     (8224, 37, 32, O.F16, True)])
@@ -24,10 +30,12 @@ def test_long_k(k, m, g, sdt, apart):
     q = np.stack([b & 15, b >> 4], 2).reshape(m, k).astype(np.float64) - 8
     s = O.to_f32(page[m * k // 2:].view(np.uint16), sdt).astype(np.float64).reshape(m, -(-k // g)).repeat(g, 1)[:, :k]
     ref = (q * s) @ xd
-    # f32: a term passes at most 40 roundings (16 of its chunk, 16 of its lane's chunks and passes, 8 of
-    # the reduction and scale), each 2^-24 of a partial sum no larger than the sum of |x| (|q - 8| + 8) s
-    # (the offset 8 is subtracted per chunk)
-    bound = 40 * 2.0 ** -24 * (((np.abs(q) + 8) * s) @ np.abs(xd))
+    # f32: the roundings a term passes, in either kernel: 31 in its chunk's offset term (32 activations
+    # added one after another; the codes' side has 16 two-term dot products over two sums, 17), 1 where the
+    # offset is subtracted, 16 multiply-adds of its lane's chunks (1024 chunks over 64 lanes), 6 of the sum
+    # over lanes, 3 of the sum over up to four waves: 57, taken as 60. Each is at most 2^-24 of a partial
+    # sum no larger than the sum of |x| (|q - 8| + 8) s.
+    bound = 60 * 2.0 ** -24 * (((np.abs(q) + 8) * s) @ np.abs(xd))
     dx, dp = torch.from_numpy(x.view(np.int16)).cuda(), torch.from_numpy(page).cuda()
     st = torch.cuda.current_stream().cuda_stream
     out = torch.full((m + 8,), 7.5, dtype=torch.float32, device="cuda")

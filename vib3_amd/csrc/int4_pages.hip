@@ -209,16 +209,28 @@ int launch_ragged(const GenericArgs& a, bool dual, hipStream_t s) {
 }
 
 // One flat matrix of 8192 < k, f16 activation: k_down_rows with one slot. k_int4_rows would need more
-// than four chunks per lane in registers, and k_int4_rows_ksplit, which splits k over two waves, reads
-// and converts the activation once per wave: 4096 x 14336 10.1 us there, 9.0 us here;
-// 512 x 8224 9.0 and 5.2; 7168 x 14336 14.4 either way. False where
-// the rows and scales are not one page, the staged activation exceeds 64 KB or rows exceed
-// page_magic's range.
+// than four chunks per lane in registers, and k_int4_rows_ksplit, which splits k over two or four waves,
+// reads and converts the activation once per wave: 1024 x 14336 9.4 us there, 5.1 here; 4096 x 14336 10.9 and
+// 10.2; 512 x 8224 9.4 and 4.9 (pages from HBM). False where the rows and scales are not one page,
+// the staged activation exceeds 64 KB, rows exceed page_magic's range, or the split kernel is faster
+// (us there / here):
+//   * more rows than one workgroup per CU takes, whose last workgroups run alone: 10240 x 8224 18.0 / 20.0,
+//     8192 x 14336 15.6 / 16.4 (from two full rounds on the long rows' kernel wins again: 14336 x 8224
+//     23.6 / 21.9, 12288 x 20480 32.6 / 30.0; 16384 x 16384 30.1 / 31.0 it does not);
+//   * staging an activation that one or a few rows use: 1 x 20480 5.3 / 6.6, 4 x 28672 6.5 / 7.7;
+//   * k > 20480, where two workgroups' LDS fill a CU: 5120 x 24576 18.5 / 19.4 (4096 15.7 / 14.2, 7168
+//     25.3 / 21.4), 3584 x 28672 15.5 / 16.1 (1024 10.2 / 7.8), 5120 x 30816 21.6 / 26.3.
 bool flat_down_ok(const RowsArgs& a) {
-  const int cpr = a.K / 32, pk = a.K / 2;
-  return a.x_dt == VIB3_DT_F16 && cpr > 4 * kWave && a.M < 65536 &&
-         down_rows_lds(1, cpr) <= 64 * 1024 &&
-         (const uint8_t*)a.flat0.scales == a.flat0.data + (size_t)a.M * pk;
+  const int cpr = a.K / 32, pk = a.K / 2, M = a.M;
+  if (a.x_dt != VIB3_DT_F16 || cpr <= 4 * kWave || M >= 65536 || down_rows_lds(1, cpr) > 64 * 1024 ||
+      (const uint8_t*)a.flat0.scales != a.flat0.data + (size_t)M * pk)
+    return false;
+  if (a.K <= 12288) return M <= 8192 || M >= 14336;
+  if (a.K <= 16384) return M <= 7168;
+  if (M <= 4) return false;
+  if (a.K <= 20480) return M <= 8192 || M >= 12288;
+  if (a.K <= 24576) return M <= 4096 || (M > 6144 && M <= 8192);
+  return M <= 2048;
 }
 
 int launch_flat_down(const RowsArgs& a, hipStream_t s) {
@@ -226,10 +238,12 @@ int launch_flat_down(const RowsArgs& a, hipStream_t s) {
   d.h = a.x; d.h_dt = a.x_dt; d.K = a.K; d.M = a.M; d.g = a.g; d.sdt = a.sdt; d.nslots = 1;
   d.rpp = a.M; d.magic = page_magic(a.M); d.flat = a.flat0.data;
   d.out = (float*)a.out; d.out_dt = a.out_dt;
-  const int waves = 6 * device_cus();
-  if (a.M / 4 >= waves) launch_down_rows_t<4, 4, false, true>(d, s, KTime{});
-  else if (a.M / 2 >= waves) launch_down_rows_t<2, 4, false, true>(d, s, KTime{});
-  else launch_down_rows_t<1, 4, false, true>(d, s, KTime{});
+  // as few rows per wave as make one eight-wave workgroup per CU (5120 rows of k = 8224: two per wave,
+  // 1.25 workgroups per CU, 13.9 us, four per wave 11.3)
+  const int waves = 8 * device_cus();
+  if (a.M <= waves) launch_down_rows_t<1, 4, false, true>(d, s, KTime{});
+  else if (a.M <= 2 * waves) launch_down_rows_t<2, 4, false, true>(d, s, KTime{});
+  else launch_down_rows_t<4, 4, false, true>(d, s, KTime{});
   VIB3_RETURN_LAUNCH();
 }
 
