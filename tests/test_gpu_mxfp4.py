@@ -180,10 +180,9 @@ def test_argument_errors():
 
 
 def test_graph_replay_equals_eager():
-    """The batched launch (grouping, then the one-token rows, two-token rows and matrix-core
-    chains on three streams, then the combine) captured in a HIP graph: the fork and join
-    become graph edges, and three replays with new activations, ids and weights each equal an
-    eager launch bit for bit."""
+    """A small batched launch (grouping, rows, matrix-core chain and combine on the caller's stream
+    alone; the forked forms: test_stream_forms) captured in a HIP graph: three replays with new
+    activations, ids and weights each equal an eager launch bit for bit."""
     from vib3_amd.mxfp4 import MoeMxfp4Batch
     _say("case: mxfp4 batch graph capture + replays")
     hidden, inter, E, T, k = 512, 768, 12, 24, 4
@@ -252,3 +251,82 @@ def test_wide_items_match_oracle(hidden, inter, E, T, k):
     got = _run(bank, x, ids, w)
     assert np.array_equal(got, _run(bank, x, ids, w))
     _check(got, _oracle(bank, xh, ids, w))
+
+
+# The forms a batch's chains run in (mx_streams): one stream, two (the matrix-core chain beside the row
+# paths), four (each row path and the wide items on their own too). (hidden, inter, E, T, k, experts of one
+# and two tokens added past the first E0, eager form, form in a captured graph).
+FORMS = [
+    (512, 768, 48, 24, 4, 48, 1, 1),
+    (1024, 1024, 48, 24, 4, 48, 1, 2),      # small experts: the fork only pays in a graph
+    (4096, 1536, 32, 16, 4, 32, 2, 2),
+    (4096, 3072, 64, 65, 4, 64, 4, 4),      # row paths of two chunks per lane in launches of their own
+    (6144, 4352, 48, 66, 4, 48, 4, 4),      # ... and of three
+    (2048, 1024, 24, 400, 6, 12, 1, 4),     # wide items with one- and two-token experts beside them
+    (4096, 4096, 8, 240, 8, 8, 4, 4),       # wide items of large experts
+]
+
+
+def _form(hidden, inter, E, T, k, capturing):
+    """The rule of mx_streams for 256 CUs."""
+    n = T * k
+    nbytes = 3 * 17 / 32 * hidden * inter * min(n, E)
+    wide = n // 64 * min(inter // 128, hidden // 256) > 256
+    if n <= 16 or (n >= 6 * E and not wide) or nbytes < (60e6 if capturing else 200e6):
+        return 1
+    if wide:
+        return 4
+    return 2 if n <= 256 or nbytes < 1e9 else 4
+
+
+def _form_picks(rng, E, E0, T, k):
+    """Zipf picks over the first E0 experts, one- and two-token experts among the others."""
+    from vib3_amd.mxfp4 import zipf_picks
+    ids, w = zipf_picks(T, E0, min(k, E0), s=1.1 if E0 == E and E > 8 else 0.0, seed=int(rng.integers(1 << 30)))
+    for i, e in enumerate(range(E0, E)):
+        ids[2 * i, 1] = e
+        if i % 2:
+            ids[2 * i + 1, 1] = e
+    return ids, w
+
+
+@pytest.mark.parametrize("hidden,inter,E,T,k,E0,eager,captured", FORMS)
+def test_stream_forms(hidden, inter, E, T, k, E0, eager, captured):
+    """Every form, eager and in a captured graph (where the forks and joins become graph edges): a sample
+    of tokens against the oracle, and three replays with new activations, ids and weights each equal
+    to the eager launch bit for bit, with eager work between them."""
+    from vib3_amd.mxfp4 import MoeMxfp4Batch
+    _say(f"case: mxfp4 form hidden={hidden} inter={inter} E={E} T={T} k={k}: {eager} eager, {captured} captured")
+    assert _form(hidden, inter, E, T, k, False) == eager and _form(hidden, inter, E, T, k, True) == captured
+    bank = _bank(hidden, inter, E, layer=5)
+    rng = np.random.default_rng(hidden + E)
+    dev = lambda ids, w: (torch.from_numpy(ids.view(np.int16)).cuda(), torch.from_numpy(w).cuda())  # noqa: E731
+    ids, w = _form_picks(rng, E, E0, T, k)
+    counts = np.bincount(ids.ravel(), minlength=E)
+    if E > 8:
+        assert (counts == 1).any() and (counts == 2).any() and (counts > 2).any()
+    xb, xh = _x(T, hidden, 90)
+    xb = xb.clone()
+    ib, wb = dev(ids, w)
+    g, ref = MoeMxfp4Batch(bank, T, k), MoeMxfp4Batch(bank, T, k)
+    got = g.launch(xb, ib, wb)
+    torch.cuda.synchronize()
+    got = got.view(torch.int16).cpu().numpy().view(np.uint16).copy()
+    sample = sorted({0, 1, 3, T // 2, T - 1})  # (0, 1, 3: tokens of one- and two-token experts past E0)
+    _check(got[sample], _oracle(bank, xh, ids, w, tokens=sample))
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        g.launch(xb, ib, wb)
+    torch.cuda.synchronize()
+    for r in range(3):
+        xt, _ = _x(T, hidden, 91 + r)
+        it, wt = dev(*_form_picks(rng, E, E0, T, k))
+        xb.copy_(xt), ib.copy_(it), wb.copy_(wt)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        replayed = g.out.clone()
+        _say(f"  replay {r}")
+        assert torch.equal(replayed.view(torch.int16), ref.launch(xt, it, wt).view(torch.int16))
+    del graph

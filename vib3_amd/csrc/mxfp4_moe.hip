@@ -1159,27 +1159,9 @@ static int mx_grid_items(const vib3_moe_mxfp4_batch* B) {
   return bound < cap ? bound : cap;
 }
 
-// How a batch's chains run (us per batch, one stream / two / four; Kimi shape unless said):
-//   * one: everything on the caller's stream, the row paths in one launch per phase. The fork and the
-//     joins cost the host 30 us and the GPU several, which few picks or small experts do not win back:
-//     1 token x top-8 51 / 56 / 84, 2 tokens 77 / 82 / 107, 4 tokens of 128 experts of 2048 x 768
-//     35 / 55 / 81.
-//   * two: the matrix-core chain beside the row paths (one launch per phase). 4 tokens 140 / 118 /
-//     136, 16 tokens 317 / 300 / 314, 32 tokens 468 / 438 / 447, of 2048 x 768 16 tokens 78 / 71 / 86
-//     and 64 tokens 103 / 102 / 109.
-//   * four: each row path and the wide items on streams of their own too, which pays once the
-//     one-token experts alone fill the GPU. 64 tokens 688 / 653 / 649, 128 tokens 1003 / 994 / 968.
-enum MxStreams { kMxOne, kMxTwo, kMxFour };
-static MxStreams mx_streams(const vib3_moe_mxfp4_batch* B) {
-  const int n = B->tokens * B->top_k;
-  const double bytes = 3.0 * (17.0 / 32) * B->hidden * B->inter * (n < B->num_experts ? n : B->num_experts);
-  if (n <= 16 || bytes < 200e6) return kMxOne;  // (weights of at most so many distinct experts)
-  return n <= 256 || bytes < 1e9 ? kMxTwo : kMxFour;
-}
-
 // Wide items: the most a batch can form (every expert's but its last has 64 tokens, and an expert with
-// any has more than kMxTokBlk: the launches' grid rows) and the fewest for which k_mx_group lists them: the smaller of the two phases' grids then
-// gives every CU a workgroup. With fewer, 16-token blocks win, as they spread over more CUs (18
+// any has more than kMxTokBlk: the launches' grid rows) and the fewest for which k_mx_group lists them:
+// the smaller of the two phases' grids then gives every CU a workgroup. With fewer, 16-token blocks win, as they spread over more CUs (18
 // experts, 67 tokens x top-2 at 2560 x 1792: 81 us narrow, 106 us wide; 16 experts, 489 tokens x
 // top-2 at 5376 x 4096: 590 us narrow, 277 us wide). The counts are only known on the device, and
 // launches that find no wide item still cost 12 us of a 655 us batch (64 tokens x top-8, Kimi
@@ -1192,6 +1174,40 @@ static MxWide mx_wide_items(const vib3_moe_mxfp4_batch* B) {
   const int gu = B->inter / 128, dn = B->hidden / 256, blocks = gu < dn ? gu : dn;
   if (n / kMxChunk * blocks <= device_cus()) return MxWide{0, 0};
   return MxWide{(device_cus() + blocks - 1) / blocks, n / (kMxTokBlk + 1)};
+}
+
+// How a batch's chains run (us per batch, one stream / two / four; Kimi shape unless said):
+//   * one: everything on the caller's stream, the row paths in one launch per phase. The fork and the
+//     joins cost the host 30 us and the GPU several, which few picks or small experts do not win back:
+//     1 token x top-8 51 / 56 / 84, 2 tokens 77 / 82 / 107, 4 tokens of 128 experts of 2048 x 768
+//     35 / 55 / 81, 512 tokens of 64 experts of 1024 x 512 62 / 75 / 89. Nor is there work to overlap
+//     where nearly every expert has enough tokens for the matrix cores: 8 experts of 4096 x 4096, 24
+//     tokens x top-2 61 / 75 / 81, 32 of 7168 x 2048, 24 tokens x top-8 182 / 196 / 188.
+//   * two: the matrix-core chain beside the row paths (one launch per phase). 4 tokens 140 / 118 /
+//     136, 16 tokens 317 / 300 / 314, 32 tokens 468 / 438 / 447. A replayed graph pays no host time
+//     for the fork: of 128 experts of 2048 x 768 (160 MB at most) 8 tokens 66 / 55 / 62, of 256 experts of
+//     1024 x 512 24 tokens 69 / 64 / 65, where eager launches take 65 / 59 / 74 and 67 / 67 / 80 and, with a
+//     wait after each, 75 / 74 / 98 and 78 / 78 / 101. (Below 60 MB one stream in graphs too: 4 tokens of 256
+//     experts of 1024 x 512 29 / 34 / 37.)
+//   * four: each row path and the wide items on streams of their own too, which pays once the
+//     one-token experts alone fill the GPU. 64 tokens 688 / 653 / 649, 128 tokens 1003 / 994 / 968. Wide items
+//     fork into four wherever the batch forks at all (a graph of 512 tokens over 32 experts of 2048 x 768
+//     110 / - / 97).
+enum MxStreams { kMxOne, kMxTwo, kMxFour };
+static bool mx_capturing(hipStream_t st) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) == hipSuccess) return cs == hipStreamCaptureStatusActive;
+  (void)hipGetLastError();  // (the null stream while another stream captures)
+  return false;
+}
+static MxStreams mx_streams(const vib3_moe_mxfp4_batch* B, const MxWide& wide, hipStream_t st) {
+  const int n = B->tokens * B->top_k, E = B->num_experts;
+  const double bytes = 3.0 * (17.0 / 32) * B->hidden * B->inter * (n < E ? n : E);
+  if (n <= 16 || (n >= 6 * E && wide.max == 0)) return kMxOne;
+  // (weights of at most so many distinct experts)
+  if (bytes < 60e6 || (bytes < 200e6 && !mx_capturing(st))) return kMxOne;
+  if (wide.max > 0) return kMxFour;
+  return n <= 256 || bytes < 1e9 ? kMxTwo : kMxFour;
 }
 
 static MxWs mx_ws(const vib3_moe_mxfp4_batch* B) {
@@ -1300,7 +1316,7 @@ int vib3_launch_moe_mxfp4_batched(const vib3_moe_mxfp4_batch* B, void* stream) {
     hipLaunchKernelGGL((k_mx_wide<false>), dim3((unsigned)(B->hidden / 256), (unsigned)wide.max),
                        dim3(256), 0, q, a);
   };
-  const MxStreams mode = wide.max > 0 ? kMxFour : mx_streams(B);
+  const MxStreams mode = mx_streams(B, wide, st);
   std::unique_lock<std::mutex> lock(g_mx_side_lock, std::defer_lock);
   MxSide* side = nullptr;
   if (mode != kMxOne) {
