@@ -330,3 +330,38 @@ def test_stream_forms(hidden, inter, E, T, k, E0, eager, captured):
         _say(f"  replay {r}")
         assert torch.equal(replayed.view(torch.int16), ref.launch(xt, it, wt).view(torch.int16))
     del graph
+
+
+def test_launch_while_another_stream_captures():
+    """The side streams belong to a capture that has forked onto them until it ends. A batch launched
+    eagerly on another stream meanwhile must run (on that stream alone) and stay out of the graph."""
+    from vib3_amd.mxfp4 import MoeMxfp4Batch, zipf_picks
+    _say("case: mxfp4 batch launched while another stream captures")
+    hidden, inter, E, T, k = 4096, 1536, 32, 16, 4  # (the two-stream form)
+    bank = _bank(hidden, inter, E, layer=6)
+    x, x2 = _x(T, hidden, 95)[0].clone(), _x(T, hidden, 96)[0]
+    picks = [tuple(torch.from_numpy(a.view(np.int16) if i == 0 else a).cuda()
+                   for i, a in enumerate(zipf_picks(T, E, k, seed=s))) for s in (1, 2, 3)]
+    a, b, ref = (MoeMxfp4Batch(bank, T, k) for _ in range(3))
+    want = [ref.launch(x, *picks[0]).clone(), ref.launch(x2, *picks[1]).clone()]
+    cap, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=cap, capture_error_mode="relaxed"):
+        a.launch(x, *picks[0])
+        with torch.cuda.stream(other):
+            b.launch(x2, *picks[1])
+    torch.cuda.synchronize()
+    assert torch.equal(b.out.view(torch.int16), want[1].view(torch.int16))  # ran at once
+    b.out.zero_()
+    for _ in range(3):
+        a.out.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(a.out.view(torch.int16), want[0].view(torch.int16))
+        assert not b.out.any()  # not in the graph
+    b.launch(x2, *picks[1])  # the side streams are free again
+    torch.cuda.synchronize()
+    assert torch.equal(b.out.view(torch.int16), want[1].view(torch.int16))
+    del graph

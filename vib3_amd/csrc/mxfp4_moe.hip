@@ -1134,6 +1134,28 @@ static MxSide* mx_side() {  // called with the lock held
   return &s;
 }
 
+// Whether the side streams can take a fork from st. One that a capture has forked onto belongs to that
+// capture until it ends: work enqueued there for another stream would become part of its graph.
+static bool mx_side_free(const MxSide& s, hipStream_t st) {
+  auto capture_of = [](hipStream_t q, bool& active) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(q, &cs, &id) != hipSuccess) {
+      (void)hipGetLastError();  // (the null stream while another stream captures)
+      cs = hipStreamCaptureStatusNone;
+    }
+    active = cs != hipStreamCaptureStatusNone;
+    return id;
+  };
+  bool mine, held;
+  const unsigned long long id = capture_of(st, mine);
+  for (hipStream_t q : {s.st, s.st2, s.st3}) {
+    const unsigned long long other = capture_of(q, held);
+    if (held && !(mine && other == id)) return false;
+  }
+  return true;
+}
+
 struct MxWs {
   size_t d_expert, d_off, d_cnt, nd, it_d, it_p0, it_np, nitems, ent_tok, ent_slot, c_dix, ncold, ncold1,
       h, d, total;
@@ -1322,6 +1344,7 @@ int vib3_launch_moe_mxfp4_batched(const vib3_moe_mxfp4_batch* B, void* stream) {
   if (mode != kMxOne) {
     lock.lock();
     side = mx_side();
+    if (side && !mx_side_free(*side, st)) side = nullptr;
     if (!side) lock.unlock();
   }
   hipError_t e = hipSuccess;
