@@ -104,7 +104,7 @@ def test_scalar(k, m):
 # rows of each lane count, pairs and tiled pages earlier than single row-major ones; rows that are no
 # whole workgroup, a staged activation near the longest the f32-input form takes.
 CHOICE = [(64, 64), (1024, 65), (1056, 64), (1056, 65), (1024, 16), (2048, 2560), (2048, 2576), (2560, 6144), (2560, 6161),
-          (4096, 6160), (3072, 12288), (3072, 12304), (4160, 6144), (4160, 6160), (4160, 8208), (4128, 12289),
+          (4096, 6160), (3072, 10241), (3072, 12288), (3072, 12304), (4160, 6144), (4160, 6160), (4160, 8208), (4128, 12289),
           (20032, 6160)]
 
 

@@ -435,16 +435,18 @@ PageShape page_shape(int M, int G) {
 //   * many rows, where the row kernel's waves walk several row groups: K = 2048 2064 rows 4.6 / 4.3,
 //     8192 5.4 / 5.7, pairs 5.5 / 5.3 and 5.7 / 6.0 (3072 rows); K = 2560 7168 rows 5.9 / 5.9, 16384
 //     7.8 / 9.3; K = 4096 12288 rows 10.2 / 9.2, 16384 10.8 / 11.4, pairs of 6144 9.9 / 9.0, 8192 10.6 / 10.8;
-//     K = 7168 12288 rows 16.3 / 14.6, pairs of 8192 16.4 / 16.4, 10240 18.6 / 19.7;
+//     K = 7168 12288 rows 16.3 / 14.6, pairs of 8192 16.4 / 16.4, 10240 18.6 / 19.7; full scales K = 3072 10240
+//     rows 7.1 / 7.1, 12288 7.4 / 8.1, K = 5120 12288 rows 10.8 / 12.3;
 //   * tiled pages, whose 64 lanes per row (K > 4096) take 32 bytes of each 128-byte line, earlier:
 //     K = 7168 6144 rows 12.2 / 12.0, 7168 12.8 / 13.2, 12288 16.4 / 21.6.
-bool page_staged(int lay, int ns, int K, int M) {
+bool page_staged(int lay, bool full, int ns, int K, int M) {
+  const int single = full ? 10240 : 12288;
   if (K <= 1024) return ns == 1 || M > 64;
   if (K <= 2048) return M > 2560;
   if (K <= 2560) return M > 6144;
-  if (K <= 4096) return M > (ns == 2 ? 6144 : 12288);
+  if (K <= 4096) return M > (ns == 2 ? 6144 : single);
   if (K >= 8192 && lay != kLayTiled) return ns == 1 && M > 14336;
-  return M > (lay == kLayTiled ? 6144 : ns == 2 ? 8192 : 12288);
+  return M > (lay == kLayTiled ? 6144 : ns == 2 ? 8192 : single);
 }
 
 int page_gemv(int lay, bool full, int ns, const void* act, const void* act_sc, const float* x,
@@ -467,7 +469,7 @@ int page_gemv(int lay, bool full, int ns, const void* act, const void* act_sc, c
   a.w[1] = (const uint8_t*)w1; a.s[1] = (const uint16_t*)s1;
   a.out = (float*)out; a.K = K; a.M = M;
   hipStream_t st = (hipStream_t)stream;
-  if (act && page_staged(lay, ns, K, M)) {
+  if (act && page_staged(lay, full, ns, K, M)) {
 #define VIB3_PAGE_STAGED(LY, F, N)                                                              \
   hipLaunchKernelGGL((k_fp4_page_staged<LY, F, N>), dim3((unsigned)((M + 15) / 16)), dim3(256), \
                      (unsigned)G * 68u, st, a)
