@@ -1,8 +1,7 @@
 // down_rows.h — k_down_rows, the down projection from activations staged in LDS, and its launch: the
 // layer's (int4_gemv.hip) and, with FLAT, a single page's (int4_pages.hip). A header, so that each
 // translation unit holds only its own instantiations: the layer's kernels are sensitive to what is
-// placed beside them (with the page kernels in int4_gemv.hip the Kimi layer took 49.8 instead of
-// 49.4 us).
+// placed beside them (with the page kernels in int4_gemv.hip the Kimi layer took about 0.5 us more).
 #pragma once
 
 #include "common.h"

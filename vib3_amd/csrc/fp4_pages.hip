@@ -45,7 +45,7 @@ struct PageGemvArgs {
   int K, M;
 };
 
-// How both kernels split a page (one launch reads at most a few megabytes, so they are bound by
+// How k_fp4_page_rows and k_nvfp4_scalar_rows split a page (one launch reads at most a few megabytes, so they are bound by
 // the round trips of a launch, not by bandwidth: every load a wave needs goes out at once, and the
 // page is spread over as many waves as it has row groups).
 //   * A row is read by L lanes, R = 64 / L rows by a wave; lane `sub` of a row takes the 32-value
@@ -58,8 +58,7 @@ struct PageGemvArgs {
 //     and 56 dependent steps per lane.)
 //   * Waves stride over the row groups, the next group's weights loading while one is reduced.
 // Traced: 520-row gate/up page pair at K = 7168 (4.2 MB) 12.2 -> 5.1 us (f32 input quantized in the
-// kernel: 36.7 -> 6.8), 1820-row down page at K = 2048 (2.1 MB) 4.9 -> 4.2 us, a pair of 14336 rows
-// at K = 4096 (66 MB) 19.6 -> 14.1 us.
+// kernel: 36.7 -> 6.8), 1820-row down page at K = 2048 (2.1 MB) 4.9 -> 4.2 us.
 constexpr int kJ = 4;
 
 // Bytes of group g of row r in layout LAY.

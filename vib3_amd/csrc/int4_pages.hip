@@ -1,8 +1,8 @@
 // int4_pages.hip — INT4 pages one at a time (the launcher API) in the shapes that k_int4_rows
 // (int4_gemv.hip) does not take at its rate: rows that are not 16-byte aligned, and k > 8192.
 //
-// k_int4_ragged — one page with any k >= 32 (odd k too) and unaligned rows; g a multiple of 32.
-// k_down_rows   — (down_rows.h, FLAT) one page with k > 8192 and an f16 activation.
+// k_int4_ragged — one page with unaligned rows of any k > 64 (odd k too); g a multiple of 32.
+// k_down_rows   — (down_rows.h, FLAT) one page with k > 8192 and an f16 activation, where flat_down_ok.
 #include "common.h"
 #include "down_rows.h"
 #include "kernels.h"
